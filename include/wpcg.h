@@ -180,15 +180,18 @@ int wpcg_linear_matvec_multi(int n, wpcg_linear* const* lins, const float* const
  * X: M rows of in_f values, contiguous, fp32 (x_dtype WPCG_DTYPE_F32) or
  * bf16 bit patterns (WPCG_DTYPE_BF16); Y: M rows of out_f floats. With
  * M == 1 and fp32 X this is wpcg_linear_matvec in the linear's mode. Else
- * the matrix-core kernel runs (64 rows of X per launch pair): the codes
- * are exact, X is rounded to bf16 (exact when given as bf16), each block's
+ * the matrix-core kernels run (one up to 64 rows of X, another, every row
+ * in one launch, above): the codes are exact, X is rounded to bf16 (exact when given as bf16), each block's
  * dots accumulate in fp32 and its scale and zero point are applied in fp32
  * (the weights are never rounded). The first batched call on a linear
  * allocates its workspace (about 16 KiB per 128 inputs plus the split-K
- * partials); make it before capturing a graph that contains the call.
+ * partials); make it before capturing a graph that contains the call. The
+ * first one with more than 64 rows of X (SPLIT: 32) also allocates the
+ * packed X of 2048 (SPLIT: 1024) rows, 4 KiB times the inputs; captured
+ * before that, such a call runs in passes of 64 rows, with the same result.
  * WPCG_DTYPE_F32_SPLIT: fp32 X fed to the matrix cores as two bf16 terms
  * hi = bf16(x), lo = bf16(x - hi), so X is carried to a relative 2^-18
- * (32 rows of X per launch; twice the matrix-core work). */
+ * (twice the matrix-core work). */
 #define WPCG_DTYPE_F32  0
 #define WPCG_DTYPE_BF16 1
 #define WPCG_DTYPE_F32_SPLIT 2
@@ -215,7 +218,7 @@ int wpcg_linear_gemm_noalloc(wpcg_linear* lin, const void* x_dev, int x_dtype, u
                              wpcg_stream stream);
 /* K-slices of the batched kernels (0 = the library's choice; a tuning knob,
  * no reference counterpart), applied to both (M <= 16 and M > 16) within
- * their limits. Frees the workspace; the next batched call makes it. The
+ * their limits; while it is set, more than 64 rows of X run 64 at a time. Frees the workspace; the next batched call makes it. The
  * query returns the splits in use (or planned) for M <= 16 and M > 16. */
 int wpcg_linear_set_gemm_kslices(wpcg_linear* lin, int kslices);
 int wpcg_linear_gemm_kslices(wpcg_linear* lin, int* kslices_small, int* kslices);

@@ -230,3 +230,39 @@ def test_gemm_split_every_ksplit(ctx, M):
         check(Y, X, 4, blocks, rows, cols, TOL_SPLIT, None, f"split kg={kg}")
         assert rel_to_max(Y, X, 4, blocks, rows, cols) <= SPLIT_REL
     lin.close()
+
+
+# The many-row kernel at the edges of its tiles: one row more than the
+# 64 (SPLIT 32) that k_gemm takes, ragged last tiles of 32 rows of X and of
+# W, odd and even block counts on both sides of the K groups (1, 2, 4, 8), and
+# every workgroup shape (outputs from one tile to more than the chip).
+# 2^-17 and 3e-5 of the term sum as in the bounds above.
+@pytest.mark.parametrize("scheme,rows,cols,M", [
+    (4, 1, 128, 65), (3, 33, 256, 95), (4, 16, 384, 96), (3, 300, 1152, 129), (4, 700, 1280, 100),
+    (3, 4864, 896, 300), (4, 9728, 640, 500), (3, 2560, 2560, 97), (4, 513, 4224, 1025), (4, 8192, 256, 2080)])
+@pytest.mark.parametrize("dtype", [wpcg.DTYPE_BF16, wpcg.DTYPE_F32, wpcg.DTYPE_F32_SPLIT])
+def test_gemm_many_rows(ctx, scheme, rows, cols, M, dtype):
+    print(f"[gpu] gemm v{scheme} {rows}x{cols} M={M} dtype={dtype}", flush=True)
+    rng = np.random.default_rng(rows + M)
+    bias = rng.standard_normal(rows).astype(np.float32)
+    lin, blocks = make(ctx, scheme, rows, cols, rows + cols, bias)
+    X = rng.standard_normal((M, cols)).astype(np.float32)
+    bits = to_bf16_bits(X)
+    Y = lin.gemm(bits if dtype == wpcg.DTYPE_BF16 else X, dtype)
+    split = dtype == wpcg.DTYPE_F32_SPLIT
+    check(Y, X if split else bf16_to_f32(bits), scheme, blocks, rows, cols, TOL_SPLIT if split else TOL_ACC, bias,
+          f"M={M}")
+    assert np.array_equal(Y.view(np.uint32), lin.gemm(bits if dtype == wpcg.DTYPE_BF16 else X, dtype).view(np.uint32))
+    # captured before the packed X of this size exists: smaller passes, the same bits
+    other, _ = make(ctx, scheme, rows, cols, rows + cols, bias)
+    xd = ctx.upload(bits if dtype == wpcg.DTYPE_BF16 else X)
+    yd = ctx.alloc(4 * M * rows)
+    other.gemm_dev(xd, 2, yd, dtype)  # the 64-column workspace
+    g = ctx.capture(lambda: other.gemm_dev(xd, M, yd, dtype))
+    for _ in range(2):
+        yd.write(np.full(M * rows, np.nan, np.float32))
+        g.launch()
+        ctx.sync()
+        assert np.array_equal(yd.read(np.float32, M * rows).view(np.uint32), Y.reshape(-1).view(np.uint32))
+    lin.close()
+    other.close()

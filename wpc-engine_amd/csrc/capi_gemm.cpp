@@ -14,6 +14,8 @@ void free_gemm(GemmWork& w)
     if (w.xsum) (void)hipFree(w.xsum);
     if (w.part) (void)hipFree(w.part);
     if (w.counters) (void)hipFree(w.counters);
+    if (w.wxf) (void)hipFree(w.wxf);
+    if (w.wxsum) (void)hipFree(w.wxsum);
     const int req = w.kg_req;
     w = GemmWork{};
     w.kg_req = req;
@@ -45,6 +47,42 @@ int make_gemm(wpcg_linear* L, hipStream_t s)
     return WPCG_OK;
 }
 
+// Whether the many-row kernel takes a batch of M rows: more than one
+// launch_gemm covers, unless the caller set the K-slices (its knob is that
+// kernel's).
+bool wide(const wpcg_linear* L, int x_mode, uint32_t M)
+{
+    return L->gemm.kg_req == 0 && M > (uint32_t)(x_mode == GX_SPLIT ? GEMM_MAX_M_SPLIT : GEMM_MAX_M) &&
+           L->m.nb * GEMM_WIDE_TILES * 4096 < (1ull << 30);  // the kernel's buffer offsets
+}
+
+// The many-row kernel over M rows. Its packed X is allocated by the first
+// such call; while a graph is being captured (no allocation) the 64-column
+// workspace serves in smaller passes, with the same results.
+int run_wide(wpcg_linear* L, const void* x, int x_mode, uint32_t M, const float* res, float* y, hipStream_t s)
+{
+    const DeviceMatrix& m = L->m;
+    GemmWork& w = L->gemm;
+    if (!w.wxf) {
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        WPCG_HIP(hipStreamIsCapturing(s, &st));
+        if (st != hipStreamCaptureStatusNone) {
+            WPCG_HIP(launch_gemm_wide(m, w.xf, w.xsum, GEMM_MAX_M / 16, x, x_mode, M, L->bias, res, y, s));
+            return WPCG_OK;
+        }
+        void* f = nullptr;
+        hipError_t e = hipMalloc(&f, m.nb * GEMM_WIDE_TILES * 4096);
+        if (e == hipSuccess) e = hipMalloc(&w.wxsum, m.nb * GEMM_WIDE_TILES * 16 * sizeof(float));
+        if (e != hipSuccess) {
+            if (f) (void)hipFree(f);
+            return hip_fail(e, "batched GEMM workspace");
+        }
+        w.wxf = f;
+    }
+    WPCG_HIP(launch_gemm_wide(m, w.wxf, w.wxsum, GEMM_WIDE_TILES, x, x_mode, M, L->bias, res, y, s));
+    return WPCG_OK;
+}
+
 int run_gemm(wpcg_linear* L, const void* x, int x_dtype, uint32_t M, float* y, hipStream_t s)
 {
     const DeviceMatrix& m = L->m;
@@ -64,6 +102,7 @@ int run_gemm(wpcg_linear* L, const void* x, int x_dtype, uint32_t M, float* y, h
                                     "make it before capturing a graph");
         if (int rc = make_gemm(L, s)) return rc;
     }
+    if (wide(L, x_dtype, M)) return run_wide(L, x, x_dtype, M, nullptr, y, s);
     const uint64_t es = x_dtype == WPCG_DTYPE_BF16 ? 2 : 4;
     const uint32_t step = x_dtype == WPCG_DTYPE_F32_SPLIT ? GEMM_MAX_M_SPLIT : GEMM_MAX_M;
     for (uint32_t c = 0; c < M; c += step) {
@@ -75,28 +114,6 @@ int run_gemm(wpcg_linear* L, const void* x, int x_dtype, uint32_t M, float* y, h
 }
 
 }  // namespace
-
-int linear_gemm(wpcg_linear* L, const float* x, int x_mode, uint32_t M, const float* res, float* y, hipStream_t s)
-{
-    const DeviceMatrix& m = L->m;
-    if (M == 0 || m.rows == 0) return WPCG_OK;
-    if (m.nb == 0) return fail(WPCG_E_SHAPE, "batched GEMM of a matrix without inputs");
-    if (!L->gemm.xf) {
-        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-        WPCG_HIP(hipStreamIsCapturing(s, &st));
-        if (st != hipStreamCaptureStatusNone)
-            return fail(WPCG_E_ARG, "the first batched call on a linear allocates its workspace: "
-                                    "make it before capturing a graph");
-        if (int rc = make_gemm(L, s)) return rc;
-    }
-    const uint32_t step = x_mode == GX_SPLIT ? GEMM_MAX_M_SPLIT : GEMM_MAX_M;
-    for (uint32_t c = 0; c < M; c += step) {
-        const int mc = (int)std::min<uint32_t>(step, M - c);
-        WPCG_HIP(launch_gemm(m, L->gemm, x + (uint64_t)c * m.cols, x_mode, mc, L->bias,
-                             res ? res + (uint64_t)c * m.rows : nullptr, y + (uint64_t)c * m.rows, s));
-    }
-    return WPCG_OK;
-}
 
 namespace {
 
@@ -158,6 +175,13 @@ int wpcg_linear_gemm_noalloc(wpcg_linear* L, const void* x, int x_dtype, uint32_
     w.xsum = reinterpret_cast<float*>(base + o_xsum);
     w.xf = base + o_xf;
     w.part = part ? reinterpret_cast<float*>(base + o_part) : nullptr;
+    if (wide(L, x_dtype, M)) {  // as many 16-column tiles as the array holds packed, a multiple of 4
+        const uint64_t room = WPCG_NOALLOC_SCRATCH_BYTES - up(ncnt * sizeof(uint32_t));
+        const int tiles = (int)std::min<uint64_t>(GEMM_WIDE_TILES, room / (m.nb * (4096 + 64)) / 4 * 4);
+        w.xf = base + o_xsum + up(m.nb * tiles * 64);
+        WPCG_HIP(launch_gemm_wide(m, w.xf, w.xsum, tiles, x, x_dtype, M, L->bias, nullptr, y, s));
+        return WPCG_OK;
+    }
     // the array keeps the last call's contents: the counters must start at 0
     WPCG_HIP(launch_fill_u32(w.counters, (int)ncnt, 0u, s));
     const uint64_t es = x_dtype == WPCG_DTYPE_BF16 ? 2 : 4;

@@ -211,6 +211,8 @@ struct GemmWork {
     float* xsum = nullptr;          // per-block column sums: nb * 64
     float* part = nullptr;          // partial Y: [kg][64][rows_pad] or [kg_small][16][rows_pad]
     uint32_t* counters = nullptr;   // one per row group, self-resetting
+    void* wxf = nullptr;            // the many-row kernel's packed X: nb * GEMM_WIDE_TILES tiles * 4 KiB
+    float* wxsum = nullptr;         // its column sums: nb * GEMM_WIDE_TILES * 16
 };
 void free_gemm(GemmWork& w);  // keeps kg_req
 int gemm_row_groups(uint64_t rows);        // more than 16 columns
@@ -226,6 +228,16 @@ constexpr int GX_F32 = 0, GX_BF16 = 1, GX_SPLIT = 2;
 constexpr int GEMM_MAX_M_SPLIT = 32;
 hipError_t launch_gemm(const DeviceMatrix& m, const GemmWork& w, const void* x, int x_mode, int M,
                        const float* bias, const float* res, float* y, hipStream_t s);
+// More rows of X than one launch_gemm takes (gemm_wide.hip): X is packed in
+// passes of gemm_wide_cols(x_mode, tiles) rows into `tiles` 16-column tiles
+// of xf / xsum, then one launch covers every row of the pass. An output
+// does not depend on the passes it is split into.
+constexpr int GEMM_WIDE_TILES = 128;  // 2048 rows of X a pass, 1024 in the SPLIT mode
+inline int gemm_wide_cols(int x_mode, int tiles) { return x_mode == GX_SPLIT ? tiles / 4 * 32 : tiles / 2 * 32; }
+hipError_t launch_gemm_wide(const DeviceMatrix& m, void* xf, float* xsum, int tiles, const void* x, int x_mode,
+                            uint32_t M, const float* bias, const float* res, float* y, hipStream_t s);
+hipError_t launch_gemm_pack(const void* x, int x_mode, int M, int K, int xt, int nt, void* xf, float* xsum,
+                            hipStream_t s);
 // Expert-grouped GEMM, one launch for every expert of a stack (or of two
 // stacks of one shape over the same X: m2 and y2, else null): m is one
 // expert's shape, its planes the first of the stack (expert e at e * its
@@ -418,9 +430,6 @@ hipError_t launch_pf_group(const int32_t* ids, int P, int E, int top_k, int* pai
                            int* nitems, hipStream_t s);
 hipError_t launch_pf_combine(float* X, const float* D, const float* w, const int* pair_pos, int T, int top_k, int H,
                              hipStream_t s);
-// Y = X W^T (+ res) for M rows of fp32 X with the linear's batched kernels
-// (x_mode GX_*), its workspace made on first use (not under capture).
-int linear_gemm(wpcg_linear* L, const float* x, int x_mode, uint32_t M, const float* res, float* y, hipStream_t s);
 // The same from the keys a FAST GEMV's workgroups left (GemvJob::amax), one
 // per workgroup in row order: a row's key is (its value's order-preserving
 // bits, -0 read as +0) << 32 | ~row, 0 for a value that does not beat -inf
