@@ -38,7 +38,6 @@ struct Prefill {
     float *ge = nullptr, *ue = nullptr, *de = nullptr;  // per sorted pair: [P][moe_inter] x2, [P][hidden]
     void* xf = nullptr;       // packed X of the batched GEMMs (launch_gemm_pack_rows)
     float* xsum = nullptr;
-    float* part = nullptr;    // K-slice partials of o_proj / the dense down
     int cus = 0;              // the device's CUs: the expert-grouped GEMMs' workgroups
     void* dg = nullptr;       // the expert-grouped GEMMs' X digits (launch_pf_digits)
     float* dxs = nullptr;
@@ -373,10 +372,15 @@ int enqueue_step(wpcg_model* m, hipStream_t s)
 }
 
 // ---- batched prefill (FAST) --------------------------------------------------
-// Rows of tokens per prefill pass; longer prompts run pass after pass.
-constexpr uint32_t PF_CAP = 256;
-constexpr int PF_MAX_KG = 4;  // K-slices of the prefill's hidden-size GEMMs
-static_assert(PF_CAP <= (uint32_t)PF_GROUP_MAXT, "the expert grouping holds PF_GROUP_MAXT tokens");
+// Rows of tokens per prefill pass; longer prompts run pass after pass. The
+// expert grouping holds PF_GROUP_MAXT tokens; a dense pass reads every
+// weight once for four times as many (the 19456 x 2560 gate and up of 1000
+// tokens: 4 x 87 us in passes of 256, 208 in one).
+constexpr uint32_t PF_CAP_DENSE = 1024;
+uint32_t pf_cap(const wpcg_model_config& c)
+{
+    return std::min(c.n_experts ? (uint32_t)PF_GROUP_MAXT : PF_CAP_DENSE, c.max_pos);
+}
 
 // Whether the batched path covers this model: FAST attention's head shapes,
 // and for MoE the router width, the pair count and one-slice expert GEMMs.
@@ -385,7 +389,7 @@ bool prefill_ok(const wpcg_model* m)
     const wpcg_model_config& c = m->cfg;
     if (!attention_fast_ok((int)c.n_heads, (int)c.n_kv_heads, (int)c.head_dim)) return false;
     if (!c.n_experts) return true;
-    const uint32_t cap = std::min(PF_CAP, c.max_pos);
+    const uint32_t cap = pf_cap(c);
     return c.n_experts <= (uint32_t)ROUTE_MAXN && cap * c.top_k <= (uint32_t)PF_MAX_PAIRS &&
            c.hidden / 128 <= (uint32_t)GEMM_GROUP_MAXBK && c.moe_inter / 128 <= (uint32_t)GEMM_GROUP_MAXBK &&
            pad_rows(c.hidden) <= (uint64_t)GEMM_GROUP_MAXROWS && pad_rows(c.moe_inter) <= (uint64_t)GEMM_GROUP_MAXROWS &&
@@ -398,7 +402,7 @@ int make_prefill(wpcg_model* m)
     if (P.cap) return WPCG_OK;
     const wpcg_model_config& c = m->cfg;
     WPCG_HIP(hipDeviceGetAttribute(&P.cus, hipDeviceAttributeMultiprocessorCount, m->ctx->device));
-    const size_t cap = std::min(PF_CAP, c.max_pos), H = c.hidden, qd = (size_t)c.n_heads * c.head_dim,
+    const size_t cap = pf_cap(c), H = c.hidden, qd = (size_t)c.n_heads * c.head_dim,
                  kvd = (size_t)c.n_kv_heads * c.head_dim;
     int rc = WPCG_OK;
     auto dev = [&](void** p, size_t bytes) {
@@ -419,7 +423,6 @@ int make_prefill(wpcg_model* m)
     const size_t kmax = std::max<size_t>({H, qd, c.n_experts ? 0 : (size_t)c.inter});
     dev((void**)&P.xf, kmax / 128 * gemm_rows_tiles((int)cap) * 4096);
     dev((void**)&P.xsum, kmax / 128 * gemm_rows_tiles((int)cap) * 16 * 4);
-    dev((void**)&P.part, (size_t)PF_MAX_KG * (gemm_rows_tiles((int)cap) / 4 * 32) * pad_rows(H) * 4);
     if (c.n_experts) {
         const size_t pairs = cap * c.top_k, E = c.n_experts, I = c.moe_inter;
         dev((void**)&P.r, cap * E * 4);
@@ -441,16 +444,6 @@ int make_prefill(wpcg_model* m)
     }
     if (rc == WPCG_OK) P.cap = (uint32_t)cap;
     return rc;
-}
-
-// K-slices of a packed-rows GEMM of the prefill whose rows are the hidden
-// size (o_proj, the dense down): enough for about 256 workgroups, slices of
-// at least 8 blocks (o_proj of the Qwen3-30B-A3B shape at 256 rows: 128
-// workgroups of 32 blocks took 26.3 us, 256 of 16 plus the slice sum ~18).
-int pf_kslices(const DeviceMatrix& m, int n)
-{
-    const int live = gemm_row_groups(m.rows) * (gemm_rows_tiles(n) / 4);
-    return std::max(1, std::min({256 / std::max(live, 1), (int)m.nb / 8, PF_MAX_KG}));
 }
 
 // Tokens tokens[pos0 .. pos0+n-1] (already on the device) through every
@@ -478,40 +471,38 @@ int prefill_pass(wpcg_model* m, uint32_t pos0, uint32_t n, hipStream_t s)
             float* ys[3] = {P.q, P.k, P.v};
             GemmRope rope{{GEMM_ROPE_Q, GEMM_ROPE_K, GEMM_ROPE_V}, {nullptr, kc, vc}, {L.q_norm, L.k_norm, nullptr},
                           m->cos_t, m->sin_t, (int)pos0, (int)c.max_pos, c.eps};
-            WPCG_HIP(launch_gemm_packed_rows_multi(ms, bs, ys, 3, P.xf, P.xsum, (int)n, s, qk_fused ? &rope : nullptr));
+            WPCG_HIP(launch_gemm_packed_rows(ms, bs, ys, 3, P.xf, P.xsum, (int)n, nullptr, s, qk_fused ? &rope : nullptr));
         }
         WPCG_HIP(launch_prefill_attention(P.q, P.k, P.v, L.q_norm, L.k_norm, nh, nkv, hd, c.eps, scale, m->cos_t,
                                           m->sin_t, (int)pos0, (int)n, (int)c.max_pos, kc, vc, P.attn, P.xf, P.xsum,
                                           s, qk_fused));
         // residual += o_proj(attn); 128-wide heads leave the attention packed
         if (hd != 128) WPCG_HIP(launch_gemm_pack_rows(P.attn, (int)n, nh * hd, P.xf, P.xsum, s));
-        // o_proj in K-slices; for the MoE model the slice sum joins the
-        // post-attention RMSNorm (the router and the experts read fp32 rows)
-        const int okg = pf_kslices(L.o->m, (int)n);
-        const bool fuse_norm = c.n_experts && okg > 1 && H <= PF_NORM_MAXH;
-        WPCG_HIP(launch_gemm_packed_rows(L.o->m, P.xf, P.xsum, (int)n, L.o->bias, P.x, P.x, s, okg, P.part,
-                                         !fuse_norm));
+        auto residual = [&](const wpcg_linear* l) {
+            const DeviceMatrix* ms[1] = {&l->m};
+            const float* bs[1] = {l->bias};
+            float* ys[1] = {P.x};
+            return launch_gemm_packed_rows(ms, bs, ys, 1, P.xf, P.xsum, (int)n, P.x, s);
+        };
+        WPCG_HIP(residual(L.o));
         if (!c.n_experts) {
             WPCG_HIP(launch_rms_pack_rows(P.x, L.post_ln, (int)n, H, c.eps, P.xf, P.xsum, s));
             const DeviceMatrix* ms[2] = {&L.gate->m, &L.up->m};
             const float* bs[2] = {L.gate->bias, L.up->bias};
             float* ys[2] = {P.g, P.u};
-            WPCG_HIP(launch_gemm_packed_rows_multi(ms, bs, ys, 2, P.xf, P.xsum, (int)n, s));
+            WPCG_HIP(launch_gemm_packed_rows(ms, bs, ys, 2, P.xf, P.xsum, (int)n, nullptr, s));
             WPCG_HIP(launch_silu_mul(P.g, P.u, P.g, (size_t)n * c.inter, s));
             WPCG_HIP(launch_gemm_pack_rows(P.g, (int)n, (int)c.inter, P.xf, P.xsum, s));
-            WPCG_HIP(launch_gemm_packed_rows(L.down->m, P.xf, P.xsum, (int)n, L.down->bias, P.x, P.x, s,
-                                             pf_kslices(L.down->m, (int)n), P.part));
+            WPCG_HIP(residual(L.down));
             continue;
         }
         // experts: route every row, sort the (row, slot) pairs by expert, one
         // grouped launch for gate and up and one for down, then the ordered
         // combine
-        // (the fused slice sum + norm also writes the experts' X digits)
-        const bool digits_done = fuse_norm && H % 128 == 0;
-        if (fuse_norm)
-            WPCG_HIP(launch_pf_reduce_norm(P.part, okg, (int)n, H, (int)L.o->m.rows_pad, L.o->bias, P.x, L.post_ln,
-                                           c.eps, P.xn, digits_done ? P.dg : nullptr,
-                                           digits_done ? P.dxs : nullptr, s));
+        // (the norm also writes the experts' X digits)
+        const bool digits_done = H % 128 == 0 && H <= PF_NORM_MAXH;
+        if (digits_done)
+            WPCG_HIP(launch_pf_norm_digits(P.x, (int)n, H, L.post_ln, c.eps, P.xn, P.dg, P.dxs, s));
         else
             WPCG_HIP(launch_rms_norm_rows(F, P.x, L.post_ln, H, (int)n, c.eps, P.xn, s));
         wpcg_moe* E = L.moe;
@@ -580,7 +571,9 @@ int verify_run(wpcg_model* m, uint32_t pos0, uint32_t n)
     if (int rc = prefill_pass(m, pos0, n, s)) return rc;
     wpcg_linear* head = logits_head(m);
     WPCG_HIP(launch_rms_pack_rows(P.x, m->final_norm, (int)n, (int)c.hidden, c.eps, P.xf, P.xsum, s));
-    WPCG_HIP(launch_gemm_packed_rows(head->m, P.xf, P.xsum, (int)n, head->bias, nullptr, P.vlogits, s));
+    const DeviceMatrix* ms[1] = {&head->m};
+    const float* bs[1] = {head->bias};
+    WPCG_HIP(launch_gemm_packed_rows(ms, bs, &P.vlogits, 1, P.xf, P.xsum, (int)n, nullptr, s));
     WPCG_HIP(launch_argmax_rows(P.vlogits, (int)c.vocab, (int)n, P.vids, s));
     WPCG_HIP(hipStreamSynchronize(s));
     uint32_t last = 0;

@@ -129,22 +129,6 @@ __global__ __launch_bounds__(256) void k_gemm_pack(const void* __restrict__ X, i
     }
 }
 
-// Another matrix of a launch that shares X (and K) with the first: its
-// workgroups start at wg0 (a multiple of 8, so each matrix's row groups keep
-// their XCDs).
-struct GemmMat {
-    const uint8_t* codes;
-    const uint8_t* hp;
-    const uint32_t* params;
-    float* y;
-    const float* bias;
-    int rows, rows_pad, rgs, rgs8, wg0;
-    int rope;            // GEMM_ROPE_*: the prefill's q, k or v epilogue
-    float* cache;        // k, v: the layer's cache [head][max_pos][128]
-    const float* nw;     // q, k: the head norm's weights [128]
-};
-constexpr int GEMM_MAX_MATS = 3;
-static_assert(GEMM_MAX_MATS == sizeof(GemmRope::mode) / sizeof(int), "GemmRope holds every matrix of a launch");
 struct GemmArgs {
     const uint8_t* codes;
     const uint8_t* hp;
@@ -156,21 +140,6 @@ struct GemmArgs {
     const float* res;    // [M][rows] added to Y (may be y itself) or null
     float* part;         // [kg][NT*16][rows_pad] (kg > 1), summed by k_gemm_reduce
     int rows, rows_pad, nb, M, kg;
-    // column groups: the packed X holds xt tiles per block (groups of NT);
-    // with rgs8 > 0 workgroup cg * rgs8 + rg takes row group rg (< rgs) of
-    // column group cg, kg = 1 (the groups of one row group share an XCD's L2)
-    int xt, rgs, rgs8;
-    int nmore;  // further matrices over the same X (rgs8 > 0 only)
-    GemmMat more[GEMM_MAX_MATS - 1];
-    // the prefill's q/k/v epilogue (GemmRope): this matrix's mode, cache and
-    // norm weights, and the rotation tables of every matrix
-    int rope;
-    float* cache;
-    const float* nw;
-    const float* cos_t;  // [max_pos][64]
-    const float* sin_t;
-    int pos0, max_pos;
-    float eps;
 };
 
 // The value written for output (m, row): the sum, the bias, the residual.
@@ -212,78 +181,6 @@ __device__ __forceinline__ bf16x8 codes_bf16(uint32_t a, uint32_t b)
 // zero point of the offset codes: zp - 128 * scale
 __device__ __forceinline__ float zp_off(uint32_t p) { return __builtin_fmaf(-128.0f, h2f(p >> 16), h2f(p & 0xFFFFu)); }
 
-// The prefill's q/k/v epilogue (kg = 1, a row group of 8 waves x 16 rows =
-// one 128-wide head, 32 columns = tokens mcol0 ..): q and k get the head
-// RMSNorm (FAST: the squares of each lane's four rows by fused multiply-adds,
-// the lane groups by exchanges, the eight waves through LDS in a fixed
-// order; then (x * scale) * w) and the rotation at each token's position
-// (rows d < 64 and d + 64 are a pair: y c - y' s and y' c + y s, as
-// fa_norm_rope). The normed rows are staged in LDS as [token][d] and leave
-// as whole 16-byte pieces of a token's row (thread t: token t / 16, rows
-// 4 (t % 16) .. +3 and the same + 64): q into Y, k and v (v as computed)
-// into the cache rows of their position. The bias is added first.
-template <typename Acc>
-__device__ __forceinline__ void rope_epilogue(const GemmArgs& P, const Acc& acc, int rg, int wave, int g, int j,
-                                              int mcol0, float* ex)
-{
-    constexpr int TOK = 32, EXS = 132;  // ex: [TOK][EXS], rows 16-byte aligned
-    float* rsum = ex + TOK * EXS;       // [8][TOK] sums of squares
-    const int mode = P.rope;
-    float v[2][4];
-#pragma unroll
-    for (int n = 0; n < 2; n++)
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int d = wave * 16 + 4 * g + q;
-            v[n][q] = acc[0][n][q] + (P.bias ? P.bias[rg * 128 + d] : 0.0f);
-        }
-    __syncthreads();  // every wave is done with the X buffers
-    float sc[2] = {1.0f, 1.0f};
-    if (mode != GEMM_ROPE_V) {
-#pragma unroll
-        for (int n = 0; n < 2; n++) {
-            float ss = fmaf(v[n][3], v[n][3], fmaf(v[n][2], v[n][2], fmaf(v[n][1], v[n][1], v[n][0] * v[n][0])));
-            ss += __shfl_xor(ss, 16);
-            ss += __shfl_xor(ss, 32);
-            if (g == 0) rsum[wave * TOK + n * 16 + j] = ss;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int n = 0; n < 2; n++) {
-            const float* r = rsum + n * 16 + j;
-            const float tot = ((r[0] + r[TOK]) + (r[2 * TOK] + r[3 * TOK])) +
-                              ((r[4 * TOK] + r[5 * TOK]) + (r[6 * TOK] + r[7 * TOK]));
-            sc[n] = __fdiv_rn(1.0f, __builtin_sqrtf(__fadd_rn(__fdiv_rn(tot, 128.0f), P.eps)));
-        }
-    }
-#pragma unroll
-    for (int n = 0; n < 2; n++)
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int d = wave * 16 + 4 * g + q;
-            ex[(n * 16 + j) * EXS + d] = mode != GEMM_ROPE_V ? (v[n][q] * sc[n]) * P.nw[d] : v[n][q];
-        }
-    __syncthreads();
-    const int tok = threadIdx.x >> 4, d1 = 4 * (threadIdx.x & 15), m = mcol0 + tok;
-    if (m >= P.M) return;
-    const int pos = P.pos0 + m;
-    const float4 y1 = *reinterpret_cast<const float4*>(&ex[tok * EXS + d1]);
-    const float4 y2 = *reinterpret_cast<const float4*>(&ex[tok * EXS + d1 + 64]);
-    float4 o1 = y1, o2 = y2;
-    if (mode != GEMM_ROPE_V) {
-        const float4 c = *reinterpret_cast<const float4*>(P.cos_t + (size_t)pos * 64 + d1);
-        const float4 sn = *reinterpret_cast<const float4*>(P.sin_t + (size_t)pos * 64 + d1);
-        o1 = make_float4(fmaf(y1.x, c.x, -(y2.x * sn.x)), fmaf(y1.y, c.y, -(y2.y * sn.y)),
-                         fmaf(y1.z, c.z, -(y2.z * sn.z)), fmaf(y1.w, c.w, -(y2.w * sn.w)));
-        o2 = make_float4(fmaf(y2.x, c.x, y1.x * sn.x), fmaf(y2.y, c.y, y1.y * sn.y), fmaf(y2.z, c.z, y1.z * sn.z),
-                         fmaf(y2.w, c.w, y1.w * sn.w));
-    }
-    float* dst = mode == GEMM_ROPE_Q ? P.y + (size_t)m * P.rows + rg * 128
-                                     : P.cache + ((size_t)rg * P.max_pos + pos) * 128;
-    *reinterpret_cast<float4*>(dst + d1) = o1;
-    *reinterpret_cast<float4*>(dst + d1 + 64) = o2;
-}
-
 // A workgroup of 8 waves (two per SIMD, so one wave's waits are filled by the
 // other's work) computes one row group (8 row tiles) for all NT*16 columns
 // over one K-slice. Wave w takes GM_RT tiles from rg*8 + w*GM_RT and every
@@ -307,7 +204,7 @@ __device__ __forceinline__ void rope_epilogue(const GemmArgs& P, const Acc& acc,
 // of the same NT/2 column tiles (k_gemm_pack<*, true>); after the loop the
 // wave adds each lo tile's sums to its hi tile's and writes the hi tiles.
 template <int SCHEME, int NT, bool SPLIT>
-__global__ __launch_bounds__(GM_WG) void k_gemm(const GemmArgs P0)
+__global__ __launch_bounds__(GM_WG) void k_gemm(const GemmArgs P)
 {
     static_assert(!SPLIT || NT % 2 == 0, "split needs hi and lo tiles");
     constexpr int RT = GM_RT;
@@ -319,41 +216,8 @@ __global__ __launch_bounds__(GM_WG) void k_gemm(const GemmArgs P0)
     __shared__ __align__(16) u32x4 xb[2][GM_R * FW];
     __shared__ float xsb[2][SN];
 
-    // this workgroup's matrix (uniform)
-    GemmArgs P = P0;
-    int bid = (int)blockIdx.x;
-    for (int e = P0.nmore - 1; e >= 0; e--)
-        if (bid >= P0.more[e].wg0) {
-            const GemmMat& mm = P0.more[e];
-            P.codes = mm.codes;
-            P.hp = mm.hp;
-            P.params = mm.params;
-            P.y = mm.y;
-            P.bias = mm.bias;
-            P.rows = mm.rows;
-            P.rows_pad = mm.rows_pad;
-            P.rgs = mm.rgs;
-            P.rgs8 = mm.rgs8;
-            P.rope = mm.rope;
-            P.cache = mm.cache;
-            P.nw = mm.nw;
-            bid -= mm.wg0;
-            break;
-        }
-    const int kg = P.kg, nb = P.nb, XT = P.xt;
-    int kgi, rg, cg;
-    if (P.rgs8) {  // workgroup (kgi * ncg + cg) * rgs8 + rg
-        const int ncg = P.xt / NT;
-        rg = bid % P.rgs8;
-        cg = (bid / P.rgs8) % ncg;
-        kgi = bid / P.rgs8 / ncg;
-        if (rg >= P.rgs) return;  // padding of the row groups, uniform
-    } else {
-        kgi = bid % kg;
-        rg = bid / kg;
-        cg = 0;
-    }
-    const int mcol0 = cg * (SPLIT ? NT / 2 : NT) * 16;  // the group's first output column
+    const int kg = P.kg, nb = P.nb;
+    const int kgi = blockIdx.x % kg, rg = blockIdx.x / kg;
     const int nbk = (nb + kg - 1) / kg;
     const int b0 = min(kgi * nbk, nb);
     const int nbl = max(0, min(nb, b0 + nbk) - b0);
@@ -373,8 +237,8 @@ __global__ __launch_bounds__(GM_WG) void k_gemm(const GemmArgs P0)
                            ok && SCHEME == 3 ? nbl * (int)HP_REC : 0);
         prs[rt] = buf_rsrc(P.params + rec * TILE_ROWS, ok ? nbl * TILE_ROWS * 4 : 0);
     }
-    const auto xrs = buf_rsrc(P.xf + ((size_t)b0 * XT + cg * NT) * 256, (nbl * XT - cg * NT) * 4096);
-    const auto srs = buf_rsrc(P.xsum + (size_t)b0 * XT * 16 + cg * NT * 16, (nbl * XT - cg * NT) * 64);
+    const auto xrs = buf_rsrc(P.xf + (size_t)b0 * NT * 256, nbl * NT * 4096);
+    const auto srs = buf_rsrc(P.xsum + (size_t)b0 * NT * 16, nbl * NT * 64);
 
     u32x4 cr[GM_LA][RT], pr[GM_LA][RT];
     u32x2 hr[GM_LA][RT];
@@ -396,13 +260,13 @@ __global__ __launch_bounds__(GM_WG) void k_gemm(const GemmArgs P0)
 #pragma unroll
         for (int v = 0; v < XV; v++) {
             const int i = min((int)threadIdx.x + v * GM_WG, GM_R * FW - 1);
-            xr[v] = __builtin_amdgcn_raw_buffer_load_b128(xrs, ((r * GM_R + i / FW) * XT * 256 + i % FW) * 16, 0, 0);
+            xr[v] = __builtin_amdgcn_raw_buffer_load_b128(xrs, (r * GM_R * FW + i) * 16, 0, 0);
         }
 #pragma unroll
         for (int v = 0; v < SV; v++) {
             const int i = min((int)threadIdx.x + v * GM_WG, SN - 1);
             sr[v] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                srs, ((r * GM_R + i / (NT * 16)) * XT * 16 + i % (NT * 16)) * 4, 0, 0));
+                srs, (r * SN + i) * 4, 0, 0));
         }
     };
     // Every thread stores every word it loaded: a thread past the end holds
@@ -563,21 +427,14 @@ __global__ __launch_bounds__(GM_WG) void k_gemm(const GemmArgs P0)
     // the column tiles this wave writes: [0, NW) (SPLIT: the hi tiles)
     constexpr int NW = SPLIT ? NT / 2 : NT;
 
-    // lane (g, j) holds rows 4g..4g+3 of each tile for column n*16 + j;
-    // the split-K partials have Mp columns (every column group's with rgs8)
-    const int Mp = P.rgs8 ? P.xt / NT * NW * 16 : NT * 16;
-    if constexpr (SPLIT && RT == 1 && NW == 2) {
-        if (P.rope) {  // uniform: the row group is one 128-wide head
-            rope_epilogue(P, acc, rg, wave, g, j, mcol0, reinterpret_cast<float*>(&xb[0][0]));
-            return;
-        }
-    }
+    // lane (g, j) holds rows 4g..4g+3 of each tile for column n*16 + j
+    constexpr int Mp = NT * 16;  // columns of the split-K partials
     if (kg == 1) {
 #pragma unroll
         for (int rt = 0; rt < RT; rt++)
 #pragma unroll
             for (int n = 0; n < NW; n++) {
-                const int m = mcol0 + n * 16 + j, row = (T0 + rt) * TILE_ROWS + 4 * g;
+                const int m = n * 16 + j, row = (T0 + rt) * TILE_ROWS + 4 * g;
                 if (m >= P.M) continue;
 #pragma unroll
                 for (int q = 0; q < 4; q++)
@@ -598,7 +455,7 @@ __global__ __launch_bounds__(GM_WG) void k_gemm(const GemmArgs P0)
     for (int rt = 0; rt < RT; rt++)
 #pragma unroll
         for (int n = 0; n < NW; n++) {
-            const int m = mcol0 + n * 16 + j, row = (T0 + rt) * TILE_ROWS + 4 * g;
+            const int m = n * 16 + j, row = (T0 + rt) * TILE_ROWS + 4 * g;
             if (T0 + rt < ntiles) {
                 u32x4 v;
                 __builtin_memcpy(&v, &acc[rt][n], 16);
@@ -1379,7 +1236,6 @@ hipError_t launch_gemm(const DeviceMatrix& m, const GemmWork& w, const void* x, 
     a.nb = nb;
     a.M = M;
     a.kg = w.kg;
-    a.xt = ntiles;
     dim3 grid((unsigned)(gemm_row_groups(m.rows) * w.kg));
     if (split) e = m.scheme == 4 ? launch_nt<4, true>(ntiles, grid, s, a) : launch_nt<3, true>(ntiles, grid, s, a);
     else e = m.scheme == 4 ? launch_nt<4, false>(ntiles, grid, s, a) : launch_nt<3, false>(ntiles, grid, s, a);
@@ -1393,108 +1249,6 @@ hipError_t launch_gemm(const DeviceMatrix& m, const GemmWork& w, const void* x, 
 hipError_t launch_gemm_pack_rows(const float* x, int M, int K, void* xf, float* xsum, hipStream_t s)
 {
     return launch_gemm_pack(x, GX_SPLIT, M, K, gemm_rows_tiles(M), 4, xf, xsum, s);
-}
-
-hipError_t launch_gemm_packed_rows(const DeviceMatrix& m, const void* xf, const float* xsum, int M, const float* bias,
-                                   const float* res, float* y, hipStream_t s, int kg, float* part, bool reduce)
-{
-    if (M < 1 || m.nb == 0 || kg < 1 || kg > (int)m.nb || (kg > 1 && !part)) return hipErrorInvalidValue;
-    (void)hipGetLastError();
-    GemmArgs a{};
-    a.codes = m.codes;
-    a.hp = m.hp;
-    a.params = m.params;
-    a.xf = static_cast<const u32x4*>(xf);
-    a.xsum = xsum;
-    a.y = y;
-    a.bias = bias;
-    a.res = res;
-    a.rows = (int)m.rows;
-    a.rows_pad = (int)m.rows_pad;
-    a.nb = (int)m.nb;
-    a.M = M;
-    a.kg = kg;
-    a.part = part;
-    a.xt = gemm_rows_tiles(M);
-    a.rgs = gemm_row_groups(m.rows);
-    a.rgs8 = (a.rgs + 7) / 8 * 8;
-    dim3 grid((unsigned)(a.rgs8 * (a.xt / 4) * kg));
-    hipError_t e = m.scheme == 4 ? launch_nt<4, true>(4, grid, s, a) : launch_nt<3, true>(4, grid, s, a);
-    if (e != hipSuccess || kg == 1 || !reduce) return e;
-    const int Mp = a.xt / 4 * 32, outs = M * (int)(m.rows_pad / 4);
-    hipLaunchKernelGGL(k_gemm_reduce, dim3((unsigned)((outs + 255) / 256)), dim3(256), 0, s, part, kg, Mp,
-                       (int)m.rows_pad, (int)m.rows, M, bias, res, y);
-    return hipGetLastError();
-}
-
-hipError_t launch_gemm_packed_rows_multi(const DeviceMatrix* const* ms, const float* const* biases, float* const* ys,
-                                         int count, const void* xf, const float* xsum, int M, hipStream_t s,
-                                         const GemmRope* rope)
-{
-    if (M < 1 || count < 1 || count > GEMM_MAX_MATS) return hipErrorInvalidValue;
-    for (int e = 0; e < count; e++)
-        if (ms[e]->nb == 0 || ms[e]->nb != ms[0]->nb || ms[e]->scheme != ms[0]->scheme) return hipErrorInvalidValue;
-    if (rope) {  // whole 128-row heads; q and k have norm weights, k and v a cache
-        if (!rope->cos_t || !rope->sin_t || rope->pos0 < 0 || rope->pos0 + M > rope->max_pos)
-            return hipErrorInvalidValue;
-        for (int e = 0; e < count; e++) {
-            const int md = rope->mode[e];
-            if (md < 0 || md > GEMM_ROPE_V || (md && ms[e]->rows % 128) || (md && md != GEMM_ROPE_V && !rope->nw[e]) ||
-                ((md == GEMM_ROPE_K || md == GEMM_ROPE_V) && !rope->cache[e]))
-                return hipErrorInvalidValue;
-        }
-    }
-    (void)hipGetLastError();
-    const DeviceMatrix& m = *ms[0];
-    GemmArgs a{};
-    a.codes = m.codes;
-    a.hp = m.hp;
-    a.params = m.params;
-    a.xf = static_cast<const u32x4*>(xf);
-    a.xsum = xsum;
-    a.y = ys[0];
-    a.bias = biases[0];
-    if (rope) {
-        a.rope = rope->mode[0];
-        a.cache = rope->cache[0];
-        a.nw = rope->nw[0];
-        a.cos_t = rope->cos_t;
-        a.sin_t = rope->sin_t;
-        a.pos0 = rope->pos0;
-        a.max_pos = rope->max_pos;
-        a.eps = rope->eps;
-    }
-    a.rows = (int)m.rows;
-    a.rows_pad = (int)m.rows_pad;
-    a.nb = (int)m.nb;
-    a.M = M;
-    a.kg = 1;
-    a.xt = gemm_rows_tiles(M);
-    a.rgs = gemm_row_groups(m.rows);
-    a.rgs8 = (a.rgs + 7) / 8 * 8;
-    int wgs = a.rgs8 * (a.xt / 4);
-    a.nmore = count - 1;
-    for (int e = 1; e < count; e++) {
-        GemmMat& mm = a.more[e - 1];
-        mm.codes = ms[e]->codes;
-        mm.hp = ms[e]->hp;
-        mm.params = ms[e]->params;
-        mm.y = ys[e];
-        mm.bias = biases[e];
-        mm.rows = (int)ms[e]->rows;
-        mm.rows_pad = (int)ms[e]->rows_pad;
-        mm.rgs = gemm_row_groups(ms[e]->rows);
-        mm.rgs8 = (mm.rgs + 7) / 8 * 8;
-        mm.wg0 = wgs;
-        if (rope) {
-            mm.rope = rope->mode[e];
-            mm.cache = rope->cache[e];
-            mm.nw = rope->nw[e];
-        }
-        wgs += mm.rgs8 * (a.xt / 4);
-    }
-    const dim3 grid((unsigned)wgs);
-    return m.scheme == 4 ? launch_nt<4, true>(4, grid, s, a) : launch_nt<3, true>(4, grid, s, a);
 }
 
 hipError_t launch_pf_digits(const float* x, const float* xu, int rows, int K, void* dg, float* dxs, hipStream_t s)

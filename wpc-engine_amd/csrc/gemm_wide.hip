@@ -1,7 +1,8 @@
 // Batched dequant-GEMM Y = X W^T for many rows of X (prompts, large decode
-// batches): gemm.hip's arithmetic (the integer codes as the exact bf16
-// values 128 + code, each block's scale and zero point in fp32, X as packed
-// bf16 or as hi + lo bf16 terms, xpack.h) on v_mfma_f32_32x32x16_bf16.
+// batches): gemm.hip's arithmetic (the integer codes exact in bf16, each
+// block's scale and zero point in fp32, X as packed bf16 or as hi + lo bf16
+// terms, xpack.h) on v_mfma_f32_32x32x16_bf16. It serves wpcg_linear_gemm
+// above 64 rows of X and every projection of the prefill.
 //
 // k_gemm re-unpacks a matrix's codes for every 64 (SPLIT: 32) rows of X and
 // pays a pack and a reduce launch for each; here one launch covers every
@@ -22,7 +23,9 @@
 // between vector and matrix phases 160-197.
 //
 // Measured, us a call, before -> now: 15360 x 3840 v4 at 1024 rows of bf16
-// 384 -> 128, 9728 x 2560 v3 at 777 rows SPLIT 541 -> 90.
+// 384 -> 135, 9728 x 2560 v3 at 777 rows SPLIT 541 -> 92; in the prefill
+// (Qwen3-4B shape, 1000 tokens, per layer) gate and up 350 -> 208, q/k/v
+// 142 -> 76, o and down 310 -> 200.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -52,28 +55,59 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void* base, int
 }
 constexpr int PAST = 1 << 30;  // added to a buffer offset: past every range, reads zero (ranges are shorter)
 
-struct WideArgs {
+// One matrix of a launch: its tiles are t0 .. t0 + rgs * cgs - 1.
+struct WideMat {
     const uint8_t* codes;
     const uint8_t* hp;
     const uint32_t* params;
-    const u32x4* xf;    // packed X, [nb][xt][4][64] fragments
-    const float* xsum;  // [nb][xt*16]
     float* y;           // [M][rows]
     const float* bias;  // [rows] or null
-    const float* res;   // [M][rows] added to Y (may be y itself) or null
-    int rows, rows_pad, nb, M, xt, rgs, cgs;
+    int rows, rows_pad, rgs, t0;
+    int rope;         // GEMM_ROPE_*: the prefill's q, k or v epilogue
+    float* cache;     // k, v: the layer's cache [head][max_pos][128]
+    const float* nw;  // q, k: the head norm's weights [128]
+};
+constexpr int WIDE_MATS = sizeof(GemmRope::mode) / sizeof(int);
+struct WideArgs {
+    WideMat mat[WIDE_MATS];
+    const u32x4* xf;    // packed X, [nb][xt][4][64] fragments
+    const float* xsum;  // [nb][xt*16]
+    const float* res;   // [M][rows] added to Y (may be y itself) or null (one matrix only)
+    int nmat, nb, M, xt, cgs, total;
+    // rope: the rotation tables and positions of the rows of X
+    const float* cos_t;  // [max_pos][64]
+    const float* sin_t;
+    int pos0, max_pos;
+    float eps;
 };
 
-// eight codes (one byte each, < 128) as the bf16 values 128 + code
+// Eight codes, one byte each, as bf16. v4: a byte 0..15 is the fp8 (e4m3)
+// number code * 2^-9 (subnormal below 8), so the fp8 conversion scaled by
+// 2^9 gives the code itself, two an instruction, and the sums carry no
+// offset (15360 x 3840 at 1024 rows of bf16: error against float64 1.6e-6
+// with 128 + code, 1.5e-7 with the codes, at the same time). v3 (codes to 63): 128 +
+// code, whose bit patterns are 0x4300 | code, one byte permute for two; the
+// products are then D + 128 S and the zero point zp - 128 scale.
+constexpr float code_offset(int scheme) { return scheme == 4 ? 0.0f : 128.0f; }
+template <int SCHEME>
 __device__ __forceinline__ bf16x8 codes_bf16(uint32_t a, uint32_t b)
 {
-    u32x4 r;
-    r.x = __builtin_amdgcn_perm(0x43434343u, a, 0x04010400u);
-    r.y = __builtin_amdgcn_perm(0x43434343u, a, 0x04030402u);
-    r.z = __builtin_amdgcn_perm(0x43434343u, b, 0x04010400u);
-    r.w = __builtin_amdgcn_perm(0x43434343u, b, 0x04030402u);
     bf16x8 o;
-    __builtin_memcpy(&o, &r, 16);
+    if constexpr (SCHEME == 4) {
+        typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+        const bf16x2 r[4] = {__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(a, 512.0f, false),
+                             __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(a, 512.0f, true),
+                             __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(b, 512.0f, false),
+                             __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(b, 512.0f, true)};
+        __builtin_memcpy(&o, r, 16);
+    } else {
+        u32x4 r;
+        r.x = __builtin_amdgcn_perm(0x43434343u, a, 0x04010400u);
+        r.y = __builtin_amdgcn_perm(0x43434343u, a, 0x04030402u);
+        r.z = __builtin_amdgcn_perm(0x43434343u, b, 0x04010400u);
+        r.w = __builtin_amdgcn_perm(0x43434343u, b, 0x04030402u);
+        __builtin_memcpy(&o, &r, 16);
+    }
     return o;
 }
 
@@ -83,8 +117,15 @@ __device__ __forceinline__ bf16x8 codes_bf16(uint32_t a, uint32_t b)
 // sums joining in group order. A round is KW blocks: its X goes through LDS
 // (two buffers, one barrier a round), fetched into registers a round ahead,
 // the codes straight into registers two rounds ahead.
-template <int SCHEME, bool SPLIT, int CT, int WR, int WC, int KW>
-__global__ __launch_bounds__(WR * WC * KW * 64, WR * WC * KW == 16 ? 4 : 2) void k_gemm_wide(const WideArgs P)
+//
+// ROPE (the prefill's q, k and v; WR % 4 == 0): four row tiles are one
+// 128-wide head. The sums go to LDS as [token][d], and 16 threads take a
+// token of a head: the head RMSNorm (FAST: squares by fused multiply-adds,
+// then exchanges), (x * scale) * w, the rotation at the token's position
+// (d < 64 and d + 64 are a pair: y c - y' s and y' c + y s), q into Y, k
+// and v (v as computed) into the cache rows, all as 16-byte pieces.
+template <int SCHEME, bool SPLIT, int CT, int WR, int WC, int KW, bool ROPE>
+__global__ __launch_bounds__(WR * WC * KW * 64, WR * WC * KW == 16 ? 4 : 2) void k_gemm_wide(const WideArgs P0)
 {
     constexpr int WG = WR * WC * KW * 64;
     constexpr int PARTS = SPLIT ? 2 : 1;
@@ -93,15 +134,24 @@ __global__ __launch_bounds__(WR * WC * KW * 64, WR * WC * KW == 16 ? 4 : 2) void
     constexpr int XV = KW * FW / WG;       // per thread and round
     static_assert(KW * FW % WG == 0, "whole words per thread");
     static_assert((KW - 1) * WR * WC * CT * 256 <= 2 * KW * FW, "the K groups' sums fit the X buffers");
-    __shared__ __align__(16) u32x4 xb[2][KW * FW];
+    static_assert(!ROPE || (WR % 4 == 0 && CT == 1), "whole heads");
+    constexpr int HS = 132;                      // floats per token of a head's stage
+    constexpr int HW = ROPE ? 32 * HS / 4 : 0;   // 16-byte words per (head, column group)
+    constexpr int XW = 2 * KW * FW > WR / 4 * C32 * HW ? 2 * KW * FW : WR / 4 * C32 * HW;
+    __shared__ __align__(16) u32x4 xw[XW];
+    u32x4* const xb[2] = {xw, xw + KW * FW};
 
     // XCD x (workgroups x, x + 8, ...) takes a contiguous run of tiles, the
     // column groups of one row group next to each other
-    const int total = P.rgs * P.cgs, per = (total + 7) / 8;
+    const int per = (P0.total + 7) / 8;
     const int t = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
-    if (t >= total) return;
-    const int rg = __builtin_amdgcn_readfirstlane(t / P.cgs), cg = t - rg * P.cgs;  // the division runs on lanes
-    const int nb = P.nb, XT = P.xt;
+    if (t >= P0.total) return;
+    int e = 0;
+    for (int i = 1; i < P0.nmat; i++) e = t >= P0.mat[i].t0 ? i : e;
+    const WideMat P = P0.mat[e];
+    const int tl = t - P.t0;
+    const int rg = __builtin_amdgcn_readfirstlane(tl / P0.cgs), cg = tl - rg * P0.cgs;  // the division runs on lanes
+    const int nb = P0.nb, XT = P0.xt;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int kw = wave / (WR * WC), wrc = wave % (WR * WC), wr = wrc / WC, wc = wrc % WC;
     const int half = lane >> 5, jj = lane & 31, j = jj & 15;
@@ -112,8 +162,8 @@ __global__ __launch_bounds__(WR * WC * KW * 64, WR * WC * KW == 16 ? 4 : 2) void
     const auto crs = buf_rsrc(P.codes + rec0 * CODE_REC, live * nb * (int)CODE_REC);
     const auto hrs = buf_rsrc((SCHEME == 3 ? P.hp : P.codes) + rec0 * HP_REC, SCHEME == 3 ? live * nb * (int)HP_REC : 0);
     const auto prs = buf_rsrc(P.params + rec0 * TILE_ROWS, live * nb * TILE_ROWS * 4);
-    const auto xrs = buf_rsrc(P.xf, nb * XT * 4096);
-    const auto srs = buf_rsrc(P.xsum, nb * XT * 64);
+    const auto xrs = buf_rsrc(P0.xf, nb * XT * 4096);
+    const auto srs = buf_rsrc(P0.xsum, nb * XT * 64);
 
     // the wave's codes of one block: word ga is lane group g = 2 ga + half of
     // 16-row tile jj / 16
@@ -197,13 +247,12 @@ __global__ __launch_bounds__(WR * WC * KW * 64, WR * WC * KW == 16 ? 4 : 2) void
             for (int ct = 0; ct < CT; ct++)
 #pragma unroll
                 for (int q = 0; q < 16; q++) D[ct][q] = 0.0f;
-            const float sc = h2f(pw[u] >> 16), z = __builtin_fmaf(-128.0f, sc, h2f(pw[u] & 0xFFFFu));
+            const float sc = h2f(pw[u] >> 16), z = __builtin_fmaf(-code_offset(SCHEME), sc, h2f(pw[u] & 0xFFFFu));
             zo = u == 1 && half == 0 ? zo : z;
             load_par(u, (r + u + 2) * KW + kw);
             const u32x4* xl = &xb[u][kw * FW + wc * CT * PARTS * 512 + lane];
-#pragma unroll
-            for (int ga = 0; ga < 2; ga++) {
-                bf16x8 W[4];
+            bf16x8 W[2][4];
+            auto unpack = [&](int ga) {
                 const u32x4 U = cw[u][ga];
                 const uint32_t MK = 0x0F0F0F0Fu;
                 u32x4 lo = {U.x & MK, U.y & MK, U.z & MK, U.w & MK};
@@ -215,22 +264,33 @@ __global__ __launch_bounds__(WR * WC * KW * 64, WR * WC * KW == 16 ? 4 : 2) void
                     hi.x |= hx & T6;        hi.y |= (hx >> 2) & T6;
                     hi.z |= hy & T6;        hi.w |= (hy >> 2) & T6;
                 }
-                W[0] = codes_bf16(lo.x, lo.y);
-                W[1] = codes_bf16(lo.z, lo.w);
-                W[2] = codes_bf16(hi.x, hi.y);
-                W[3] = codes_bf16(hi.z, hi.w);
+                W[ga][0] = codes_bf16<SCHEME>(lo.x, lo.y);
+                W[ga][1] = codes_bf16<SCHEME>(lo.z, lo.w);
+                W[ga][2] = codes_bf16<SCHEME>(hi.x, hi.y);
+                W[ga][3] = codes_bf16<SCHEME>(hi.z, hi.w);
                 load_word(u, ga, (r + u + 2) * KW + kw);
+            };
+            // part p of X against the codes of word ga. The lo terms of SPLIT
+            // go first: their sums are 2^-9 of the hi terms', so only the hi
+            // terms' products are rounded at full size.
+            auto products = [&](int p, int ga) {
 #pragma unroll
                 for (int i = 0; i < 4; i++)
 #pragma unroll
-                    for (int ct = 0; ct < CT; ct++)
-#pragma unroll
-                        for (int p = 0; p < PARTS; p++) {
-                            bf16x8 X;
-                            const u32x4 w = xl[((ct * PARTS + p) * 8 + i * 2 + ga) * 64];
-                            __builtin_memcpy(&X, &w, 16);
-                            D[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(X, W[i], D[ct], 0, 0, 0);
-                        }
+                    for (int ct = 0; ct < CT; ct++) {
+                        bf16x8 X;
+                        const u32x4 w = xl[((ct * PARTS + p) * 8 + i * 2 + ga) * 64];
+                        __builtin_memcpy(&X, &w, 16);
+                        D[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(X, W[ga][i], D[ct], 0, 0, 0);
+                    }
+            };
+            unpack(0);
+            products(PARTS - 1, 0);
+            unpack(1);
+            products(PARTS - 1, 1);
+            if constexpr (SPLIT) {
+                products(0, 0);
+                products(0, 1);
             }
 #pragma unroll
             for (int ct = 0; ct < CT; ct++)
@@ -245,7 +305,7 @@ __global__ __launch_bounds__(WR * WC * KW * 64, WR * WC * KW == 16 ? 4 : 2) void
 
     // the K groups' sums, in group order
     if constexpr (KW > 1) {
-        float* red = reinterpret_cast<float*>(&xb[0][0]);
+        float* red = reinterpret_cast<float*>(xw);
         if (kw > 0) {
 #pragma unroll
             for (int ct = 0; ct < CT; ct++)
@@ -254,18 +314,68 @@ __global__ __launch_bounds__(WR * WC * KW * 64, WR * WC * KW == 16 ? 4 : 2) void
                     red[((((kw - 1) * WR * WC + wrc) * CT + ct) * 16 + q) * 64 + lane] = acc[ct][q];
         }
         __syncthreads();
-        if (kw > 0) return;
+        if (!ROPE && kw > 0) return;
+        if (kw == 0) {
 #pragma unroll
-        for (int k = 1; k < KW; k++)
+            for (int k = 1; k < KW; k++)
 #pragma unroll
-            for (int ct = 0; ct < CT; ct++)
+                for (int ct = 0; ct < CT; ct++)
 #pragma unroll
-                for (int q = 0; q < 16; q++)
-                    acc[ct][q] += red[((((k - 1) * WR * WC + wrc) * CT + ct) * 16 + q) * 64 + lane];
+                    for (int q = 0; q < 16; q++)
+                        acc[ct][q] += red[((((k - 1) * WR * WC + wrc) * CT + ct) * 16 + q) * 64 + lane];
+        }
     }
 
     // lane (half, jj) holds weight row jj for the rows 8 (q / 4) + 4 half + q % 4 of X
     const int row = T0 * TILE_ROWS + jj;
+    if constexpr (ROPE) {
+        float* ex = reinterpret_cast<float*>(xw);
+        if constexpr (KW > 1) __syncthreads();  // the K groups' sums are read
+        if (kw == 0) {
+            const float bias = P.bias && row < P.rows ? P.bias[row] : 0.0f;
+#pragma unroll
+            for (int q = 0; q < 16; q++)
+                ex[((wr / 4 * C32 + wc) * 32 + 8 * (q >> 2) + 4 * half + (q & 3)) * HS + (wr & 3) * 32 + jj] =
+                    acc[0][q] + bias;
+        }
+        __syncthreads();
+        const int d1 = 4 * (threadIdx.x & 15);
+        for (int i = (int)threadIdx.x >> 4; i < WR / 4 * C32 * 32; i += WG / 16) {
+            const int hd = i / (C32 * 32), tok = i % (C32 * 32);
+            const int m = cg * C32 * 32 + tok, head = rg * (WR / 4) + hd;
+            const float4 y1 = *reinterpret_cast<const float4*>(&ex[i * HS + d1]);
+            const float4 y2 = *reinterpret_cast<const float4*>(&ex[i * HS + d1 + 64]);
+            float4 o1 = y1, o2 = y2;
+            // (the sixteen lanes of a token are all live: their exchanges are whole)
+            if (P.rope != GEMM_ROPE_V) {
+                float ss = fmaf(y1.w, y1.w, fmaf(y1.z, y1.z, fmaf(y1.y, y1.y, y1.x * y1.x)));
+                ss = fmaf(y2.w, y2.w, fmaf(y2.z, y2.z, fmaf(y2.y, y2.y, fmaf(y2.x, y2.x, ss))));
+                ss += __shfl_xor(ss, 1);
+                ss += __shfl_xor(ss, 2);
+                ss += __shfl_xor(ss, 4);
+                ss += __shfl_xor(ss, 8);
+                const float sc = __fdiv_rn(1.0f, __builtin_sqrtf(__fadd_rn(__fdiv_rn(ss, 128.0f), P0.eps)));
+                const int pos = min(P0.pos0 + m, P0.max_pos - 1);
+                const float4 w1 = *reinterpret_cast<const float4*>(P.nw + d1);
+                const float4 w2 = *reinterpret_cast<const float4*>(P.nw + d1 + 64);
+                const float4 c = *reinterpret_cast<const float4*>(P0.cos_t + (size_t)pos * 64 + d1);
+                const float4 sn = *reinterpret_cast<const float4*>(P0.sin_t + (size_t)pos * 64 + d1);
+                const float4 n1 = make_float4((y1.x * sc) * w1.x, (y1.y * sc) * w1.y, (y1.z * sc) * w1.z, (y1.w * sc) * w1.w);
+                const float4 n2 = make_float4((y2.x * sc) * w2.x, (y2.y * sc) * w2.y, (y2.z * sc) * w2.z, (y2.w * sc) * w2.w);
+                o1 = make_float4(fmaf(n1.x, c.x, -(n2.x * sn.x)), fmaf(n1.y, c.y, -(n2.y * sn.y)),
+                                 fmaf(n1.z, c.z, -(n2.z * sn.z)), fmaf(n1.w, c.w, -(n2.w * sn.w)));
+                o2 = make_float4(fmaf(n2.x, c.x, n1.x * sn.x), fmaf(n2.y, c.y, n1.y * sn.y),
+                                 fmaf(n2.z, c.z, n1.z * sn.z), fmaf(n2.w, c.w, n1.w * sn.w));
+            }
+            if (m < P0.M && head * 128 < P.rows) {
+                float* dst = P.rope == GEMM_ROPE_Q ? P.y + (size_t)m * P.rows + head * 128
+                                                   : P.cache + ((size_t)head * P0.max_pos + P0.pos0 + m) * 128;
+                *reinterpret_cast<float4*>(dst + d1) = o1;
+                *reinterpret_cast<float4*>(dst + d1 + 64) = o2;
+            }
+        }
+        return;
+    }
     if (row >= P.rows) return;
     const float bias = P.bias ? P.bias[row] : 0.0f;
 #pragma unroll
@@ -273,24 +383,28 @@ __global__ __launch_bounds__(WR * WC * KW * 64, WR * WC * KW == 16 ? 4 : 2) void
 #pragma unroll
         for (int q = 0; q < 16; q++) {
             const int m = ((cg * WC + wc) * CT + ct) * 32 + 8 * (q >> 2) + 4 * half + (q & 3);
-            if (m >= P.M) continue;
+            if (m >= P0.M) continue;
             float v = acc[ct][q];
             if (P.bias) v += bias;
             const size_t at = (size_t)m * P.rows + row;
-            if (P.res) v += P.res[at];
+            if (P0.res) v += P0.res[at];
             P.y[at] = v;
         }
 }
 
 
-template <int SCHEME, bool SPLIT, int CT, int WR, int WC, int KW>
+template <int SCHEME, bool SPLIT, int CT, int WR, int WC, int KW, bool ROPE = false>
 hipError_t launch_cfg(WideArgs a, hipStream_t s)
 {
-    const int tiles32 = (a.rows_pad + 31) / 32;
-    a.rgs = (tiles32 + WR - 1) / WR;
     a.cgs = ((a.M + 31) / 32 + CT * WC - 1) / (CT * WC);
-    const int total = a.rgs * a.cgs;
-    hipLaunchKernelGGL((k_gemm_wide<SCHEME, SPLIT, CT, WR, WC, KW>), dim3((unsigned)((total + 7) / 8 * 8)),
+    a.total = 0;
+    for (int e = 0; e < a.nmat; e++) {
+        WideMat& m = a.mat[e];
+        m.rgs = ((m.rows_pad + 31) / 32 + WR - 1) / WR;
+        m.t0 = a.total;
+        a.total += m.rgs * a.cgs;
+    }
+    hipLaunchKernelGGL((k_gemm_wide<SCHEME, SPLIT, CT, WR, WC, KW, ROPE>), dim3((unsigned)((a.total + 7) / 8 * 8)),
                        dim3(WR * WC * KW * 64), 0, s, a);
     return hipGetLastError();
 }
@@ -308,13 +422,14 @@ struct Shape {
     bool shared;  // workgroups of 8 waves share a CU: the chip fills by fractions of a round
 };
 
-int pick(const Shape* sh, int n, int tiles32, int cols32, int scheme)
+int pick(const Shape* sh, int n, const WideArgs& a, int cols32, int scheme)
 {
     int best = 0;
     int64_t best_t = INT64_MAX;
     for (int i = 0; i < n; i++) {
-        const int64_t wgs = (int64_t)((tiles32 + sh[i].rows32 - 1) / sh[i].rows32) *
-                            ((cols32 + sh[i].cols32 - 1) / sh[i].cols32);
+        int64_t wgs = 0;
+        for (int e = 0; e < a.nmat; e++) wgs += ((a.mat[e].rows_pad + 31) / 32 + sh[i].rows32 - 1) / sh[i].rows32;
+        wgs *= (cols32 + sh[i].cols32 - 1) / sh[i].cols32;
         const int64_t c = sh[i].cost[scheme == 3];
         const int64_t t = sh[i].shared ? std::max(c * 4 / 3 * 256, c * (wgs + 128)) : (wgs + 255) / 256 * 256 * c;
         if (t < best_t) {
@@ -325,14 +440,15 @@ int pick(const Shape* sh, int n, int tiles32, int cols32, int scheme)
     return best;
 }
 
+// M: the rows of X that pick the shape (the whole batch of a pass)
 template <int SCHEME, bool SPLIT>
-hipError_t launch_any(const WideArgs& a, uint32_t M, hipStream_t s)
+hipError_t launch_any(const WideArgs& a, uint32_t M, bool rope, hipStream_t s)
 {
-    const int tiles32 = (a.rows_pad + 31) / 32, cols32 = (int)((M + 31) / 32);
+    const int cols32 = (int)((M + 31) / 32);
     if constexpr (!SPLIT) {
         static constexpr Shape sh[] = {{8, 4, {200, 220}, false}, {4, 2, {62, 69}, true}, {4, 2, {70, 80}, false},
                                        {4, 1, {39, 60}, false}, {2, 1, {33, 57}, false}};
-        switch (pick(sh, 5, tiles32, cols32, SCHEME)) {
+        switch (pick(sh, 5, a, cols32, SCHEME)) {
         case 0: return launch_cfg<SCHEME, SPLIT, 2, 8, 2, 1>(a, s);
         case 1: return launch_cfg<SCHEME, SPLIT, 1, 4, 2, 1>(a, s);
         case 2: return launch_cfg<SCHEME, SPLIT, 1, 4, 2, 2>(a, s);
@@ -340,9 +456,20 @@ hipError_t launch_any(const WideArgs& a, uint32_t M, hipStream_t s)
         default: return launch_cfg<SCHEME, SPLIT, 1, 2, 1, 8>(a, s);
         }
     } else {
+        // (the last one has no whole heads: not for rope)
         static constexpr Shape sh[] = {{16, 1, {160, 165}, false}, {4, 2, {110, 118}, true}, {4, 2, {100, 110}, false},
                                        {4, 1, {65, 80}, false}, {8, 1, {88, 105}, false}, {2, 1, {60, 70}, false}};
-        switch (pick(sh, 6, tiles32, cols32, SCHEME)) {
+        const int c = pick(sh, rope ? 5 : 6, a, cols32, SCHEME);
+        if (rope) {
+            switch (c) {
+            case 0: return launch_cfg<SCHEME, SPLIT, 1, 16, 1, 1, true>(a, s);
+            case 1: return launch_cfg<SCHEME, SPLIT, 1, 4, 2, 1, true>(a, s);
+            case 2: return launch_cfg<SCHEME, SPLIT, 1, 4, 2, 2, true>(a, s);
+            case 3: return launch_cfg<SCHEME, SPLIT, 1, 4, 1, 4, true>(a, s);
+            default: return launch_cfg<SCHEME, SPLIT, 1, 8, 1, 2, true>(a, s);
+            }
+        }
+        switch (c) {
         case 0: return launch_cfg<SCHEME, SPLIT, 1, 16, 1, 1>(a, s);
         case 1: return launch_cfg<SCHEME, SPLIT, 1, 4, 2, 1>(a, s);
         case 2: return launch_cfg<SCHEME, SPLIT, 1, 4, 2, 2>(a, s);
@@ -351,6 +478,19 @@ hipError_t launch_any(const WideArgs& a, uint32_t M, hipStream_t s)
         default: return launch_cfg<SCHEME, SPLIT, 1, 2, 1, 4>(a, s);
         }
     }
+}
+
+WideMat wide_mat(const DeviceMatrix& m, const float* bias, float* y)
+{
+    WideMat w{};
+    w.codes = m.codes;
+    w.hp = m.hp;
+    w.params = m.params;
+    w.y = y;
+    w.bias = bias;
+    w.rows = (int)m.rows;
+    w.rows_pad = (int)m.rows_pad;
+    return w;
 }
 
 }  // namespace
@@ -371,24 +511,60 @@ hipError_t launch_gemm_wide(const DeviceMatrix& m, void* xf, float* xsum, int ti
                                         (int)m.cols, xt, split ? 4 : xt, xf, xsum, s);
         if (e != hipSuccess) return e;
         WideArgs a{};
-        a.codes = m.codes;
-        a.hp = m.hp;
-        a.params = m.params;
+        a.mat[0] = wide_mat(m, bias, y + (uint64_t)c * m.rows);
+        a.nmat = 1;
         a.xf = static_cast<const u32x4*>(xf);
         a.xsum = xsum;
-        a.y = y + (uint64_t)c * m.rows;
-        a.bias = bias;
         a.res = res ? res + (uint64_t)c * m.rows : nullptr;
-        a.rows = (int)m.rows;
-        a.rows_pad = (int)m.rows_pad;
         a.nb = (int)m.nb;
         a.M = mc;
         a.xt = xt;
-        if (split) e = m.scheme == 4 ? launch_any<4, true>(a, M, s) : launch_any<3, true>(a, M, s);
-        else e = m.scheme == 4 ? launch_any<4, false>(a, M, s) : launch_any<3, false>(a, M, s);
+        if (split) e = m.scheme == 4 ? launch_any<4, true>(a, M, false, s) : launch_any<3, true>(a, M, false, s);
+        else e = m.scheme == 4 ? launch_any<4, false>(a, M, false, s) : launch_any<3, false>(a, M, false, s);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
+}
+
+hipError_t launch_gemm_packed_rows(const DeviceMatrix* const* ms, const float* const* biases, float* const* ys,
+                                   int count, const void* xf, const float* xsum, int M, const float* res,
+                                   hipStream_t s, const GemmRope* rope)
+{
+    if (M < 1 || count < 1 || count > WIDE_MATS || (res && count > 1)) return hipErrorInvalidValue;
+    if (ms[0]->nb * (uint64_t)gemm_rows_tiles(M) * 4096 >= (uint64_t)PAST) return hipErrorInvalidValue;
+    WideArgs a{};
+    for (int e = 0; e < count; e++) {
+        if (ms[e]->nb == 0 || ms[e]->nb != ms[0]->nb || ms[e]->scheme != ms[0]->scheme) return hipErrorInvalidValue;
+        a.mat[e] = wide_mat(*ms[e], biases[e], ys[e]);
+        if (!rope) continue;
+        // whole 128-row heads; q and k have norm weights, k and v a cache
+        const int md = rope->mode[e];
+        if (md < GEMM_ROPE_Q || md > GEMM_ROPE_V || ms[e]->rows % 128 || (md != GEMM_ROPE_V && !rope->nw[e]) ||
+            (md != GEMM_ROPE_Q && !rope->cache[e]))
+            return hipErrorInvalidValue;
+        a.mat[e].rope = md;
+        a.mat[e].cache = rope->cache[e];
+        a.mat[e].nw = rope->nw[e];
+    }
+    if (rope) {
+        if (!rope->cos_t || !rope->sin_t || rope->pos0 < 0 || rope->pos0 + M > rope->max_pos)
+            return hipErrorInvalidValue;
+        a.cos_t = rope->cos_t;
+        a.sin_t = rope->sin_t;
+        a.pos0 = rope->pos0;
+        a.max_pos = rope->max_pos;
+        a.eps = rope->eps;
+    }
+    (void)hipGetLastError();
+    a.nmat = count;
+    a.xf = static_cast<const u32x4*>(xf);
+    a.xsum = xsum;
+    a.res = res;
+    a.nb = (int)ms[0]->nb;
+    a.M = M;
+    a.xt = gemm_rows_tiles(M);
+    return ms[0]->scheme == 4 ? launch_any<4, true>(a, (uint32_t)M, rope != nullptr, s)
+                              : launch_any<3, true>(a, (uint32_t)M, rope != nullptr, s);
 }
 
 }  // namespace wpcg

@@ -142,17 +142,13 @@ __global__ __launch_bounds__(256) void k_rms_pack(const float* __restrict__ X, c
     }
 }
 
-// o_proj's K-slices added in slice order with its bias and the residual into
-// X (the new residual, as k_gemm_reduce writes it), and that row's RMSNorm
-// (FAST, as k_rms_norm rows computes it: each thread's squares by fused
-// multiply-adds, the wave sums, the four waves in a fixed order) into XN:
-// one workgroup of 256 threads per row, H <= 256 * RN_MAXV. With dg, the
-// normed row also as the expert GEMM's X digits (xdigits.h; the values
-// k_pf_digits would read from XN), staged in LDS.
+// Each row's RMSNorm (FAST, as k_rms_norm rows computes it: each thread's
+// squares by fused multiply-adds, the wave sums, the four waves in a fixed
+// order) into XN: one workgroup of 256 threads per row, H <= 256 * RN_MAXV.
+// With dg, the normed row also as the expert GEMM's X digits (xdigits.h; the
+// values k_pf_digits would read from XN), staged in LDS.
 constexpr int RN_MAXV = PF_NORM_MAXH / 256;
-__global__ __launch_bounds__(256) void k_pf_reduce_norm(const float* __restrict__ part, int kg, int Mp,
-                                                        int rows_pad, int H, const float* __restrict__ bias,
-                                                        float* __restrict__ X, const float* __restrict__ w,
+__global__ __launch_bounds__(256) void k_pf_norm_digits(const float* __restrict__ X, int H, const float* __restrict__ w,
                                                         float eps, float* __restrict__ XN, uint8_t* __restrict__ dg,
                                                         float2* __restrict__ dxs)
 {
@@ -160,20 +156,14 @@ __global__ __launch_bounds__(256) void k_pf_reduce_norm(const float* __restrict_
     __shared__ float xn_s[PF_NORM_MAXH];
     __shared__ __align__(16) uint8_t rec[PF_NORM_MAXH / 128 + 1][512];  // the last: blocks past the row
     const int m = blockIdx.x;
-    const size_t slice = (size_t)Mp * rows_pad;
     float v[RN_MAXV];
     float sq = 0.0f;
 #pragma unroll
     for (int i = 0; i < RN_MAXV; i++) {
         const int k = threadIdx.x + 256 * i;
         if (k < H) {
-            const float* p = part + (size_t)m * rows_pad + k;
-            float s = p[0];
-            for (int q = 1; q < kg; q++) s = s + p[q * slice];
-            if (bias) s += bias[k];
-            s += X[(size_t)m * H + k];
-            v[i] = s;
-            sq = fmaf(s, s, sq);
+            v[i] = X[(size_t)m * H + k];
+            sq = fmaf(v[i], v[i], sq);
         }
     }
     sq = wave_sum(sq);
@@ -186,7 +176,6 @@ __global__ __launch_bounds__(256) void k_pf_reduce_norm(const float* __restrict_
         const int k = threadIdx.x + 256 * i;
         if (k < H) {
             const float xn = __fmul_rn(__fmul_rn(v[i], scale), w[k]);
-            X[(size_t)m * H + k] = v[i];
             XN[(size_t)m * H + k] = xn;
             xn_s[k] = xn;
         }
@@ -342,14 +331,13 @@ hipError_t launch_rms_pack_rows(const float* X, const float* w, int n, int H, fl
     return hipGetLastError();
 }
 
-hipError_t launch_pf_reduce_norm(const float* part, int kg, int M, int H, int rows_pad, const float* bias, float* X,
-                                 const float* w, float eps, float* XN, void* dg, float* dxs, hipStream_t s)
+hipError_t launch_pf_norm_digits(const float* X, int M, int H, const float* w, float eps, float* XN, void* dg,
+                                 float* dxs, hipStream_t s)
 {
-    if (M < 1 || kg < 1 || H < 1 || H > 256 * RN_MAXV || rows_pad < H || (dg && (H % 128 || !dxs)))
-        return hipErrorInvalidValue;
+    if (M < 1 || H < 1 || H > 256 * RN_MAXV || (dg && (H % 128 || !dxs))) return hipErrorInvalidValue;
     (void)hipGetLastError();
-    hipLaunchKernelGGL(k_pf_reduce_norm, dim3((unsigned)M), dim3(256), 0, s, part, kg, gemm_rows_tiles(M) / 4 * 32,
-                       rows_pad, H, bias, X, w, eps, XN, static_cast<uint8_t*>(dg), reinterpret_cast<float2*>(dxs));
+    hipLaunchKernelGGL(k_pf_norm_digits, dim3((unsigned)M), dim3(256), 0, s, X, H, w, eps, XN,
+                       static_cast<uint8_t*>(dg), reinterpret_cast<float2*>(dxs));
     return hipGetLastError();
 }
 

@@ -253,27 +253,20 @@ hipError_t launch_gemm_pack(const void* x, int x_mode, int M, int K, int xt, int
 constexpr int GEMM_GROUP_COLS = 16;
 constexpr int GEMM_GROUP_MAXBK = 16;
 constexpr int GEMM_GROUP_MAXROWS = 2048;
-// Many rows of fp32 X in the SPLIT mode as one launch per matrix: X packed
-// once (launch_gemm_pack_rows; the pack serves every matrix with K inputs),
-// then workgroups over (row group, group of 32 rows of X); xf holds
-// K/128 * gemm_rows_tiles(M) * 4 KiB, xsum K/128 * gemm_rows_tiles(M) * 16
-// floats.
+// Many rows of fp32 X in the SPLIT mode (gemm_wide.hip): X packed once
+// (launch_gemm_pack_rows; the pack serves every matrix with K inputs); xf
+// holds K/128 * gemm_rows_tiles(M) * 4 KiB, xsum K/128 *
+// gemm_rows_tiles(M) * 16 floats.
 inline int gemm_rows_tiles(int M) { return (M + 31) / 32 * 4; }
 hipError_t launch_gemm_pack_rows(const float* x, int M, int K, void* xf, float* xsum, hipStream_t s);
-// kg > 1: K in kg slices whose partials go to part (kg * (gemm_rows_tiles(M) /
-// 4 * 32) * m.rows_pad floats), added in slice order by a second launch
-// (reduce), or left there for launch_pf_reduce_norm (bias, res, y unused).
-hipError_t launch_gemm_packed_rows(const DeviceMatrix& m, const void* xf, const float* xsum, int M, const float* bias,
-                                   const float* res, float* y, hipStream_t s, int kg = 1, float* part = nullptr,
-                                   bool reduce = true);
 // Up to three matrices of the same K and scheme over one packed X in one
-// launch (the projections that share an input: q, k, v; gate, up); no
-// residual. With rope, matrix e's epilogue per mode[e] (128-wide heads,
-// rows % 128 == 0; M rows of X are the tokens at positions pos0 ..):
-// GEMM_ROPE_Q the head RMSNorm (weights nw[e]) and the rotation (cos_t /
-// sin_t [max_pos][64]) into Y, GEMM_ROPE_K the same into cache[e]
-// ([head][max_pos][128]), GEMM_ROPE_V the rows as computed into cache[e];
-// 0 the plain output.
+// launch (the projections that share an input: q, k, v; gate, up), or one
+// with a residual (res: [M][rows] added to Y, may be y itself). With rope,
+// matrix e's epilogue per mode[e] (128-wide heads, rows % 128 == 0; M rows
+// of X are the tokens at positions pos0 ..): GEMM_ROPE_Q the head RMSNorm
+// (weights nw[e]) and the rotation (cos_t / sin_t [max_pos][64]) into Y,
+// GEMM_ROPE_K the same into cache[e] ([head][max_pos][128]), GEMM_ROPE_V the
+// rows as computed into cache[e].
 constexpr int GEMM_ROPE_Q = 1, GEMM_ROPE_K = 2, GEMM_ROPE_V = 3;
 struct GemmRope {
     int mode[3];
@@ -284,9 +277,9 @@ struct GemmRope {
     int pos0, max_pos;
     float eps;
 };
-hipError_t launch_gemm_packed_rows_multi(const DeviceMatrix* const* ms, const float* const* biases, float* const* ys,
-                                         int count, const void* xf, const float* xsum, int M, hipStream_t s,
-                                         const GemmRope* rope = nullptr);
+hipError_t launch_gemm_packed_rows(const DeviceMatrix* const* ms, const float* const* biases, float* const* ys,
+                                   int count, const void* xf, const float* xsum, int M, const float* res,
+                                   hipStream_t s, const GemmRope* rope = nullptr);
 // The grouped GEMM's X: rows x rows of K fp32 (xu non-null: silu(x) * xu,
 // the FAST steps' arithmetic, xu of x's shape) to int8 digits, dg
 // rows * K * 4 bytes, and per 128-value block {s_b 2^-7, sum}, dxs
@@ -413,13 +406,12 @@ hipError_t launch_route_rows(const float* scores, int n, int rows, int top_k, in
 // launch_gemm_pack_rows's layout), H % 128 == 0.
 hipError_t launch_rms_pack_rows(const float* X, const float* w, int n, int H, float eps, void* xf, float* xsum,
                                 hipStream_t s);
-// A K-sliced packed-rows GEMM's partials (launch_gemm_packed_rows with
-// reduce = false) summed with bias and the residual into X [M][H], then each
-// row's FAST RMSNorm with weights w into XN; H <= PF_NORM_MAXH. dg non-null:
-// XN's rows also as launch_pf_digits writes them (dg, dxs), H % 128 == 0.
+// Each row's FAST RMSNorm with weights w of X [M][H] into XN; H <=
+// PF_NORM_MAXH. dg non-null: XN's rows also as launch_pf_digits writes them
+// (dg, dxs), H % 128 == 0.
 constexpr int PF_NORM_MAXH = 4096;
-hipError_t launch_pf_reduce_norm(const float* part, int kg, int M, int H, int rows_pad, const float* bias, float* X,
-                                 const float* w, float eps, float* XN, void* dg, float* dxs, hipStream_t s);
+hipError_t launch_pf_norm_digits(const float* X, int M, int H, const float* w, float eps, float* XN, void* dg,
+                                 float* dxs, hipStream_t s);
 // R[t][e] = X[t] . W[e] (fp32 router rows), R is [T][E].
 hipError_t launch_pf_router(const float* X, const float* W, int T, int E, int K, float* R, hipStream_t s);
 // (token, slot) pairs sorted by expert for launch_gemm_grouped: pair_tok
