@@ -176,6 +176,26 @@ def test_fast_decode_tracks_the_reference(ctx, name, cfg, n_steps, seed):
     ref.close()
 
 
+@pytest.mark.parametrize("name,cfg", [("moe", dict(MOE, max_pos=790)), ("dense-rep4", dict(DENSE, n_heads=8, max_pos=790))])
+def test_fast_steps_across_the_long_context_line(ctx, name, cfg):
+    """Steps on both sides of position 768, where the attention goes from 16
+    chunks to 64 (and a MoE model's o_proj from merging them itself to a merge
+    of its own), after a batched prompt; then back across the line. Logits
+    within FAST_TOL of the range of the oracle's, the prompt's bound 5e-5."""
+    m, ref = build(ctx, cfg, 818)
+    m.set_mode(wpcg.MODE_FAST)
+    toks = np.random.default_rng(8).integers(0, cfg["vocab"], 775).astype(np.uint32)
+    exp = [ref.forward_token(int(t)) for t in toks]
+    m.prefill(toks[:764])
+    got = [m.forward_token(int(t))[0] for t in toks[764:]]
+    m.set_position(766)
+    got += [m.forward_token(int(t))[0] for t in toks[766:770]]
+    for g, r in zip(got, exp[764:] + exp[766:770]):
+        assert float(np.max(np.abs(g - r))) <= 5e-5 * float(r.max() - r.min())
+    m.close()
+    ref.close()
+
+
 @pytest.mark.parametrize("factor,nan_rows,answers", [(2.0, (3,), (0, 70)), (0.5, (0, 3), (1, 70))])
 def test_fast_argmax_ties_and_nan(ctx, factor, nan_rows, answers):
     """The FAST head leaves one argmax key per workgroup and the argmax

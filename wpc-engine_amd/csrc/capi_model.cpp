@@ -75,9 +75,11 @@ struct wpcg_model {
     float* d2 = nullptr;
     // the FAST head's per-workgroup argmax keys (one per 16-row tile at most)
     uint64_t* amax = nullptr;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
-    int graph_mode = -1;
+    // the captured steps: [0], and [1] for positions from LONG_POS on
+    // (step_kind)
+    hipGraph_t graph[2] = {nullptr, nullptr};
+    hipGraphExec_t exec[2] = {nullptr, nullptr};
+    int graph_mode[2] = {-1, -1};
     bool use_graph = true;  // false: steps are enqueued launch by launch
     bool use_prefill = true;  // FAST: prompts go through the batched prefill
     Prefill pf;
@@ -110,10 +112,33 @@ int set_linear(wpcg_model* m, wpcg_linear** dst, const void* data, uint64_t nbyt
     return WPCG_OK;
 }
 
+void drop_graph(wpcg_model* m)
+{
+    for (int k = 0; k < 2; k++) {
+        if (m->exec[k]) (void)hipGraphExecDestroy(m->exec[k]);
+        if (m->graph[k]) (void)hipGraphDestroy(m->graph[k]);
+        m->exec[k] = nullptr;
+        m->graph[k] = nullptr;
+        m->graph_mode[k] = -1;
+    }
+}
+
+// Which step runs at a position: FAST attention over 16 chunks, or (1) over
+// 64 from LONG_POS on. A chunk's workgroup takes 32 positions at a time, ~5
+// us each, so 16 chunks of position 3000 run six in a row (Qwen3-4B shape,
+// attention and merge: 33.4 + 4.8 us a layer, with 64 chunks 13.0 + 4.1);
+// below LONG_POS the 16 chunks run one or two and cost less (a step of 4
+// such layers at 500: 213 us, with 64 chunks 218; 2 Qwen3-30B-A3B-shaped
+// ones, whose o_proj merges 16 chunks itself, 143 and 146).
+constexpr uint32_t LONG_POS = 768;
+int step_kind(const wpcg_model* m, uint32_t pos)
+{
+    return m->mode == WPCG_MODE_FAST && m->part_o && pos >= LONG_POS;
+}
+
 void free_model(wpcg_model* m)
 {
-    if (m->exec) (void)hipGraphExecDestroy(m->exec);
-    if (m->graph) (void)hipGraphDestroy(m->graph);
+    drop_graph(m);
     for (auto& L : m->layers) {
         for (wpcg_linear* l : {L.q, L.k, L.v, L.o, L.gate, L.up, L.down})
             if (l) wpcg_linear_destroy(l);
@@ -122,15 +147,6 @@ void free_model(wpcg_model* m)
     if (m->embed) wpcg_linear_destroy(m->embed);
     if (m->lm_head) wpcg_linear_destroy(m->lm_head);
     for (void* p : m->allocs) (void)hipFree(p);
-}
-
-void drop_graph(wpcg_model* m)
-{
-    if (m->exec) (void)hipGraphExecDestroy(m->exec);
-    if (m->graph) (void)hipGraphDestroy(m->graph);
-    m->exec = nullptr;
-    m->graph = nullptr;
-    m->graph_mode = -1;
 }
 
 // The logits head as the reference's loaders choose it: the dense decoder
@@ -208,7 +224,7 @@ bool defer_down(const wpcg_model* m)
 // logits, argmax, position + 1. FAST mode folds the RMSNorms into the
 // GEMVs that read them and runs the MoE layer as three launches (moe_run);
 // EXACT mode keeps every operation of the reference as its own launch.
-int enqueue_step(wpcg_model* m, hipStream_t s)
+int enqueue_step(wpcg_model* m, int kind, hipStream_t s)
 {
     const wpcg_model_config& c = m->cfg;
     const int H = (int)c.hidden, hd = (int)c.head_dim, nh = (int)c.n_heads, nkv = (int)c.n_kv_heads;
@@ -259,17 +275,18 @@ int enqueue_step(wpcg_model* m, hipStream_t s)
         float* vc = m->vc + (size_t)l * nkv * c.max_pos * hd;
         if (fast && m->part_o) {
             // chunked attention; o_proj merges the chunks, residual += o_proj(attn)
+            const int chunks = kind ? ATTN_CHUNKS_LONG : ATTN_CHUNKS;
             WPCG_HIP(launch_attention_chunks(m->q, m->k, m->v, L.q_norm, L.k_norm, nh, nkv, hd, c.eps, scale,
-                                             m->rope, (int)c.max_pos, m->st, kc, vc, m->part_o, m->part_ml, s));
+                                             m->rope, (int)c.max_pos, m->st, kc, vc, m->part_o, m->part_ml, chunks, s));
             // The dense model merges the chunks once, in a launch of its own,
             // and runs o_proj as a plain GEMV: its o_proj is unsplit (32
             // blocks per workgroup), so each of its 160 workgroups merged
             // the chunk states of every head, 43 MB of reads per launch
             // (o_proj 9.3 us; merge 2.x us + plain GEMV). The MoE model's
             // two-slice o_proj merges half the heads per workgroup and keeps
-            // the merge in its prep.
-            const bool merge_apart = !c.n_experts;
-            if (merge_apart) WPCG_HIP(launch_attention_merge(m->part_o, m->part_ml, nh, hd, m->attn, s));
+            // the merge in its prep (of 16 chunks).
+            const bool merge_apart = !c.n_experts || kind;
+            if (merge_apart) WPCG_HIP(launch_attention_merge(m->part_o, m->part_ml, nh, hd, chunks, m->attn, s));
             GemvJob o{&L.o->m, &L.o->plan, merge_apart ? m->attn : m->part_o, m->residual, m->residual};
             if (!merge_apart) {
                 o.xform = XF_MERGE;
@@ -583,14 +600,15 @@ int verify_run(wpcg_model* m, uint32_t pos0, uint32_t n)
     return WPCG_OK;
 }
 
-int ensure_graph(wpcg_model* m)
+int ensure_graph(wpcg_model* m, int kind)
 {
     if (!m->use_graph) return WPCG_OK;
-    if (m->exec && m->graph_mode == m->mode) return WPCG_OK;
-    drop_graph(m);
+    if (m->exec[kind] && m->graph_mode[kind] == m->mode) return WPCG_OK;
+    if (m->exec[0] && m->graph_mode[0] != m->mode) drop_graph(m);
+    if (m->exec[1] && m->graph_mode[1] != m->mode) drop_graph(m);
     hipStream_t s = m->ctx->stream;
     WPCG_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    const int rc = enqueue_step(m, s);
+    const int rc = enqueue_step(m, kind, s);
     hipGraph_t g = nullptr;
     const hipError_t e = hipStreamEndCapture(s, &g);
     if (rc != WPCG_OK) {
@@ -598,18 +616,27 @@ int ensure_graph(wpcg_model* m)
         return rc;
     }
     if (e != hipSuccess) return hip_fail(e, "capture of the decode step");
-    m->graph = g;
-    WPCG_HIP(hipGraphInstantiate(&m->exec, g, nullptr, nullptr, 0));
-    m->graph_mode = m->mode;
+    m->graph[kind] = g;
+    const hipError_t ie = hipGraphInstantiate(&m->exec[kind], g, nullptr, nullptr, 0);
+    if (ie != hipSuccess) {
+        (void)hipGraphDestroy(g);
+        m->graph[kind] = nullptr;
+        m->exec[kind] = nullptr;
+        return hip_fail(ie, "instantiation of the decode step");
+    }
+    m->graph_mode[kind] = m->mode;
     return WPCG_OK;
 }
 
-// One step on the context stream: the captured graph, or the launches.
-int run_step(wpcg_model* m)
+// One step at position pos on the context stream: the captured graph (made
+// by the first step that needs it), or the launches.
+int run_step(wpcg_model* m, uint32_t pos)
 {
     hipStream_t s = m->ctx->stream;
-    if (!m->use_graph) return enqueue_step(m, s);
-    WPCG_HIP(hipGraphLaunch(m->exec, s));
+    const int kind = step_kind(m, pos);
+    if (!m->use_graph) return enqueue_step(m, kind, s);
+    if (int rc = ensure_graph(m, kind)) return rc;
+    WPCG_HIP(hipGraphLaunch(m->exec[kind], s));
     return WPCG_OK;
 }
 
@@ -617,8 +644,7 @@ int ready(wpcg_model* m)
 {
     const std::string miss = missing(m);
     if (!miss.empty()) return fail(WPCG_E_ARG, "tensor not set: " + miss);
-    if (int rc = check_ctx(m->ctx)) return rc;
-    return ensure_graph(m);
+    return check_ctx(m->ctx);
 }
 
 }  // namespace
@@ -699,8 +725,8 @@ int wpcg_model_create(wpcg_ctx* ctx, int scheme, const wpcg_model_config* cfg, w
     dev((void**)&m->h, inter * 4);
     dev((void**)&m->logits, (size_t)c.vocab * 4);
     if (attention_fast_ok((int)c.n_heads, (int)c.n_kv_heads, (int)hd)) {
-        dev((void**)&m->part_o, (size_t)ATTN_CHUNKS * qd * 4);
-        dev((void**)&m->part_ml, (size_t)ATTN_CHUNKS * c.n_heads * 2 * 4);
+        dev((void**)&m->part_o, (size_t)ATTN_CHUNKS_LONG * qd * 4);
+        dev((void**)&m->part_ml, (size_t)ATTN_CHUNKS_LONG * c.n_heads * 2 * 4);
         dev((void**)&m->rope, (size_t)hd * 4);
         dev((void**)&m->amax, (size_t)(c.vocab + TILE_ROWS - 1) / TILE_ROWS * 8);
         dev((void**)&m->o2, (size_t)c.hidden * 4);
@@ -941,7 +967,7 @@ int wpcg_model_forward_token(wpcg_model* m, uint32_t token, float* logits, uint3
     st.n_prompt = 0xffffffffu;
     WPCG_HIP(hipMemcpy(m->st, &st, sizeof st, hipMemcpyHostToDevice));
     WPCG_HIP(hipMemcpy(m->tokens + st.pos, &token, 4, hipMemcpyHostToDevice));
-    if (int rc = run_step(m)) return rc;
+    if (int rc = run_step(m, st.pos)) return rc;
     WPCG_HIP(hipStreamSynchronize(s));
     if (logits) WPCG_HIP(hipMemcpy(logits, m->logits, (size_t)m->cfg.vocab * 4, hipMemcpyDeviceToHost));
     if (argmax) {
@@ -1000,13 +1026,13 @@ int wpcg_model_generate(wpcg_model* m, const uint32_t* prompt, uint32_t n_prompt
         // decode steps
         rc = prefill_run(m, 0, n_prompt, n_prompt);
         (void)hipEventRecord(e0, s);
-        for (uint32_t i = 1; i < n_new && rc == WPCG_OK; i++) rc = run_step(m);
+        for (uint32_t i = 1; i < n_new && rc == WPCG_OK; i++) rc = run_step(m, n_prompt + i - 1);
     } else {
         // steps at positions 0..n_prompt-1 consume the prompt (the last one
         // yields the first new token); the n_new-1 after it are pure decode
         for (uint32_t i = 0; i < n_prompt + n_new - 1 && rc == WPCG_OK; i++) {
             if (i == n_prompt) (void)hipEventRecord(e0, s);
-            rc = run_step(m);
+            rc = run_step(m, i);
         }
     }
     (void)hipEventRecord(e1, s);
@@ -1054,7 +1080,7 @@ int wpcg_model_prefill(wpcg_model* m, const uint32_t* tokens, uint32_t n, float*
     } else {
         WPCG_HIP(hipMemcpy(m->st, &st, sizeof st, hipMemcpyHostToDevice));
         for (uint32_t i = 0; i < n; i++)
-            if (int rc = run_step(m)) return rc;
+            if (int rc = run_step(m, pos0 + i)) return rc;
     }
     WPCG_HIP(hipStreamSynchronize(s));
     if (logits) WPCG_HIP(hipMemcpy(logits, m->logits, (size_t)m->cfg.vocab * 4, hipMemcpyDeviceToHost));
@@ -1090,7 +1116,7 @@ int wpcg_model_verify(wpcg_model* m, const uint32_t* tokens, uint32_t n, uint32_
     st.n_prompt = 0xffffffffu;
     WPCG_HIP(hipMemcpy(m->st, &st, sizeof st, hipMemcpyHostToDevice));
     for (uint32_t i = 0; i < n; i++) {
-        if (int rc = run_step(m)) return rc;
+        if (int rc = run_step(m, pos0 + i)) return rc;
         WPCG_HIP(hipStreamSynchronize(s));
         if (logits) WPCG_HIP(hipMemcpy(logits + i * V, m->logits, V * 4, hipMemcpyDeviceToHost));
         WPCG_HIP(hipMemcpy(&st, m->st, sizeof st, hipMemcpyDeviceToHost));

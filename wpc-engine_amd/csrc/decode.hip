@@ -473,10 +473,10 @@ __global__ __launch_bounds__(AT_WG) void k_attention(const float* __restrict__ q
 // ---- FAST attention step: positions split into chunks across workgroups ----
 // Workgroup (j, c) takes kv head j's query heads (n_rep = nh/nkv of them)
 // over chunk c of the n = pos + 1 positions: positions are dealt round
-// robin, chunk c holding positions c, c + FA_NCH, c + 2 FA_NCH, ..., taken
-// FA_C at a time as blocks (block b: positions c + FA_NCH (FA_C b + t),
+// robin, chunk c holding positions c, c + NCH, c + 2 NCH, ..., taken
+// FA_C at a time as blocks (block b: positions c + NCH (FA_C b + t),
 // t < FA_C). The launch has a fixed shape (a HIP graph replays it at every
-// position), no chunk holds more than ceil(n / FA_NCH) positions (the
+// position), no chunk holds more than ceil(n / NCH) positions (the
 // launch takes as long as its fullest chunk), and a chunk's first block
 // does not depend on the position: its keys and values can be requested at
 // entry, with the query rows, before the position is known (each row is
@@ -495,7 +495,6 @@ __global__ __launch_bounds__(AT_WG) void k_attention(const float* __restrict__ q
 // fused multiply-adds: deterministic, not the reference's operation order.
 // head_dim HD is 64 or 128, n_rep <= FA_MAXREP.
 constexpr int FA_C = 32;
-constexpr int FA_NCH = ATTN_CHUNKS;
 constexpr int FA_MAXREP = 16;
 
 // RMSNorm of one head row (w) then RoPE at the current position, by one
@@ -532,8 +531,8 @@ __device__ __forceinline__ void fa_norm_rope(const float* x, const float* w, flo
 // query head and so twice the bytes per speculated row, requests only the
 // rows before the position, once it is known (speculating took the dense
 // Qwen3-4B-shaped launch from 5.21 to 5.42 us).
-template <int HD, int FD_WG>
-__global__ __launch_bounds__(FD_WG) void k_attention_fast(const float* __restrict__ qp,
+template <int HD, int FD_WG, int NCH>
+__global__ __launch_bounds__(FD_WG, FD_WG == 512 ? 4 : 1) void k_attention_fast(const float* __restrict__ qp,
                                                           const float* __restrict__ kp,
                                                           const float* __restrict__ vp,
                                                           const float* __restrict__ qn,
@@ -544,7 +543,17 @@ __global__ __launch_bounds__(FD_WG) void k_attention_fast(const float* __restric
                                                           float* __restrict__ kc, float* __restrict__ vc,
                                                           float* __restrict__ part_o, float* __restrict__ part_ml)
 {
-    constexpr int HD4 = HD / 4, KS = HD + 4;  // KS: key rows 16-byte aligned, offset by 4 banks
+    // A score is one thread's (256 threads: one or more scores each), or with
+    // 512 threads (at most 128 scores a block) SP = 4 lanes': lane p takes the
+    // 16-byte pieces p, p + 4, ... of the dot, added by two exchanges (one
+    // thread a score left three quarters of the 512 idle: Qwen3-4B-shaped
+    // decode at position 500, 4 layers, 220 -> 213 us a step). The 512-thread
+    // kernel is held to 128 registers, two workgroups a CU: at 136 the 64
+    // chunks of position 3000 took 18.9 us, at 128 13.0.
+    constexpr int SP = FD_WG == 512 ? 4 : 1;
+    // KS: key rows 16-byte aligned, offset by 4 banks (SP = 4: by 16, so that
+    // the pieces of four rows' four lanes lie in different banks)
+    constexpr int HD4 = HD / 4, KS = HD + 4 * SP;
     constexpr int NOUT = FA_MAXREP * HD / FD_WG;   // outputs per thread
     constexpr int G = FD_WG / HD;                  // thread groups over head_dim
     constexpr int NKV = FA_C * HD4 / FD_WG;        // 16-byte key (and value) loads per thread and block
@@ -559,11 +568,11 @@ __global__ __launch_bounds__(FD_WG) void k_attention_fast(const float* __restric
     // where it is first used was a further dependent round trip)
     asm volatile("" ::"s"(qp), "s"(kp), "s"(vp), "s"(qn), "s"(kn), "s"(nh), "s"(nkv), "s"(rope), "s"(cache_pos),
                  "s"(st), "s"(kc), "s"(vc));
-    const int j = blockIdx.x / FA_NCH, c = blockIdx.x % FA_NCH;
+    const int j = blockIdx.x / NCH, c = blockIdx.x % NCH;
     const int n_rep = nh / nkv;
-    // row t of this chunk's block b is position base(b) + FA_NCH t
-    auto base = [&](int b) { return c + b * FA_C * FA_NCH; };
-    auto row_pos = [&](int b, int t) { return base(b) + t * FA_NCH; };
+    // row t of this chunk's block b is position base(b) + NCH t
+    auto base = [&](int b) { return c + b * FA_C * NCH; };
+    auto row_pos = [&](int b, int t) { return base(b) + t * NCH; };
     float* kb = kc + (size_t)j * cache_pos * HD;
     float* vb = vc + (size_t)j * cache_pos * HD;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -655,9 +664,9 @@ __global__ __launch_bounds__(FD_WG) void k_attention_fast(const float* __restric
         return;
     }
     // the rows of block b before n (a prefix: positions grow with t)
-    auto rows = [&](int b) { return min(FA_C, (n - base(b) + FA_NCH - 1) / FA_NCH); };
+    auto rows = [&](int b) { return min(FA_C, (n - base(b) + NCH - 1) / NCH); };
     if constexpr (!SPEC) load_block(0, rows(0));
-    const bool has_pos = (int)(pos % FA_NCH) == c;
+    const bool has_pos = (int)(pos % NCH) == c;
     {
         const int nrows = n_rep + (has_pos ? 1 : 0);
 #pragma unroll
@@ -718,13 +727,13 @@ __global__ __launch_bounds__(FD_WG) void k_attention_fast(const float* __restric
         __syncthreads();
         if (base(b + 1) < n) load_block(b + 1, rows(b + 1));  // in flight during this block
         // scores s[r][t] = (q_r . k_t) * scale
-        for (int i = threadIdx.x; i < n_rep * FA_C; i += FD_WG) {
-            const int r = i / FA_C, t = i % FA_C;
+        for (int i = (int)threadIdx.x / SP; i < n_rep * FA_C; i += FD_WG / SP) {
+            const int r = i / FA_C, t = i % FA_C, p = (int)threadIdx.x % SP;
             float dot = -INFINITY;
             if (t < nt) {
                 float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
 #pragma unroll
-                for (int d = 0; d < HD; d += 4) {
+                for (int d = 4 * p; d < HD; d += 4 * SP) {
                     const float4 q4 = *reinterpret_cast<const float4*>(&qs[r][d]);
                     const float4 k4 = *reinterpret_cast<const float4*>(&ks[t][d]);
                     a0 = fmaf(q4.x, k4.x, a0);
@@ -732,9 +741,14 @@ __global__ __launch_bounds__(FD_WG) void k_attention_fast(const float* __restric
                     a2 = fmaf(q4.z, k4.z, a2);
                     a3 = fmaf(q4.w, k4.w, a3);
                 }
-                dot = ((a0 + a1) + (a2 + a3)) * scale;
+                dot = (a0 + a1) + (a2 + a3);
+                if constexpr (SP == 4) {  // (the four lanes of a score share t: all or none are here)
+                    dot += __shfl_xor(dot, 1);
+                    dot += __shfl_xor(dot, 2);
+                }
+                dot *= scale;
             }
-            ps[r][t] = dot;
+            if (p == 0) ps[r][t] = dot;
         }
         __syncthreads();
         // running softmax per head (one wave per head, lanes = positions)
@@ -771,6 +785,7 @@ __global__ __launch_bounds__(FD_WG) void k_attention_fast(const float* __restric
                     }
             }
         } else {
+#pragma unroll 8
             for (int t = 0; t < nt; t++) {
                 const float v = vs[t][d];
 #pragma unroll
@@ -1085,31 +1100,56 @@ __global__ __launch_bounds__(256) void k_add(float* __restrict__ x, const float*
 // x, with the same operations in the same order (chunk order, fused
 // multiply-adds, one correctly rounded reciprocal), done once per head for
 // a plain GEMV that follows. Workgroup h, thread d < hd.
-__global__ __launch_bounds__(128) void k_attention_merge(const float* __restrict__ part_o,
-                                                         const float* __restrict__ part_ml, int nh, int hd,
-                                                         float* __restrict__ out)
+//
+// NCH > 16: group q of 128 threads takes chunks 16 q .. 16 q + 15 against the
+// maximum of all, and the groups' sums are added in group order (one group
+// reading 64 chunks took 9.2 us a launch, four 4.1).
+template <int NCH>
+__global__ __launch_bounds__(NCH * 8) void k_attention_merge(const float* __restrict__ part_o,
+                                                             const float* __restrict__ part_ml, int nh, int hd,
+                                                             float* __restrict__ out)
 {
-    const int h = blockIdx.x, d = threadIdx.x;
-    if (d >= hd) return;
+    constexpr int NG = NCH / 16;
+    __shared__ float sa[NG][128], sl[NG][128], sm[NG];
+    const int h = blockIdx.x, d = threadIdx.x & 127, q = threadIdx.x >> 7;
+    const bool on = d < hd;
     const size_t stride = (size_t)nh * hd;
-    float m[ATTN_CHUNKS], l[ATTN_CHUNKS], o[ATTN_CHUNKS];
+    float m[16], l[16], o[16];
 #pragma unroll
-    for (int cc = 0; cc < ATTN_CHUNKS; cc++) {
-        m[cc] = part_ml[((size_t)cc * nh + h) * 2];
-        l[cc] = part_ml[((size_t)cc * nh + h) * 2 + 1];
-        o[cc] = part_o[cc * stride + (size_t)h * hd + d];
+    for (int i = 0; i < 16; i++) {
+        const int cc = q * 16 + i;
+        m[i] = part_ml[((size_t)cc * nh + h) * 2];
+        l[i] = part_ml[((size_t)cc * nh + h) * 2 + 1];
+        o[i] = on ? part_o[cc * stride + (size_t)h * hd + d] : 0.0f;
     }
     float M = -INFINITY;
 #pragma unroll
-    for (int cc = 0; cc < ATTN_CHUNKS; cc++) M = fmaxf(M, m[cc]);
+    for (int i = 0; i < 16; i++) M = fmaxf(M, m[i]);
+    if constexpr (NG > 1) {
+        if (d == 0) sm[q] = M;
+        __syncthreads();
+#pragma unroll
+        for (int g = 0; g < NG; g++) M = fmaxf(M, sm[g]);
+    }
     float L = 0.0f, a = 0.0f;
 #pragma unroll
-    for (int cc = 0; cc < ATTN_CHUNKS; cc++) {
-        const float w = __expf(m[cc] - M);  // 0 for a chunk that held no position
-        L = fmaf(w, l[cc], L);
-        a = fmaf(w, o[cc], a);
+    for (int i = 0; i < 16; i++) {
+        const float w = __expf(m[i] - M);  // 0 for a chunk that held no position
+        L = fmaf(w, l[i], L);
+        a = fmaf(w, o[i], a);
     }
-    out[(size_t)h * hd + d] = a * __fdiv_rn(1.0f, L);
+    if constexpr (NG > 1) {
+        sl[q][d] = L;
+        sa[q][d] = a;
+        __syncthreads();
+        if (q > 0) return;
+#pragma unroll
+        for (int g = 1; g < NG; g++) {
+            L += sl[g][d];
+            a += sa[g][d];
+        }
+    }
+    if (on) out[(size_t)h * hd + d] = a * __fdiv_rn(1.0f, L);
 }
 
 // ---- argmax (sampling.rs:3-14) and the next step's input -------------------
@@ -1354,14 +1394,20 @@ hipError_t launch_attention(int mode, const float* q, const float* k, const floa
 hipError_t launch_attention_chunks(const float* q, const float* k, const float* v, const float* qn,
                                    const float* kn, int nh, int nkv, int hd, float eps, float scale,
                                    const float* rope, int cache_pos, const DecodeState* st, float* kc,
-                                   float* vc, float* part_o, float* part_ml, hipStream_t s)
+                                   float* vc, float* part_o, float* part_ml, int chunks, hipStream_t s)
 {
-    if (!attention_fast_ok(nh, nkv, hd) || !rope || cache_pos < 1 || (size_t)cache_pos * hd * 4 > 0x7fffffffu)
+    if (!attention_fast_ok(nh, nkv, hd) || !rope || cache_pos < 1 || (size_t)cache_pos * hd * 4 > 0x7fffffffu ||
+        (chunks != ATTN_CHUNKS && chunks != ATTN_CHUNKS_LONG))
         return hipErrorInvalidValue;
     (void)hipGetLastError();
-#define WPCG_ATT(HD, WG)                                                                                  \
-    hipLaunchKernelGGL((k_attention_fast<HD, WG>), dim3(nkv * FA_NCH), dim3(WG), 0, s, q, k, v, qn, kn, nh, nkv, \
-                       eps, scale, rope, cache_pos, st, kc, vc, part_o, part_ml)
+#define WPCG_ATT_N(HD, WG, NCH)                                                                               \
+    hipLaunchKernelGGL((k_attention_fast<HD, WG, NCH>), dim3(nkv * NCH), dim3(WG), 0, s, q, k, v, qn, kn, nh, \
+                       nkv, eps, scale, rope, cache_pos, st, kc, vc, part_o, part_ml)
+#define WPCG_ATT(HD, WG)                                              \
+    do {                                                              \
+        if (chunks == ATTN_CHUNKS) WPCG_ATT_N(HD, WG, ATTN_CHUNKS);   \
+        else WPCG_ATT_N(HD, WG, ATTN_CHUNKS_LONG);                    \
+    } while (0)
     const bool wide = nh / nkv <= 4;
     if (hd == 128) {
         if (wide) WPCG_ATT(128, 512);
@@ -1371,6 +1417,7 @@ hipError_t launch_attention_chunks(const float* q, const float* k, const float* 
         else WPCG_ATT(64, 256);
     }
 #undef WPCG_ATT
+#undef WPCG_ATT_N
     return hipGetLastError();
 }
 
@@ -1405,12 +1452,17 @@ hipError_t launch_prefill_attention(float* Q, const float* Kx, const float* Vx, 
     return hipGetLastError();
 }
 
-hipError_t launch_attention_merge(const float* part_o, const float* part_ml, int nh, int hd, float* out,
+hipError_t launch_attention_merge(const float* part_o, const float* part_ml, int nh, int hd, int chunks, float* out,
                                   hipStream_t s)
 {
-    if (nh < 1 || hd < 1 || hd > 128) return hipErrorInvalidValue;
+    if (nh < 1 || hd < 1 || hd > 128 || (chunks != ATTN_CHUNKS && chunks != ATTN_CHUNKS_LONG))
+        return hipErrorInvalidValue;
     (void)hipGetLastError();
-    hipLaunchKernelGGL(k_attention_merge, dim3(nh), dim3(128), 0, s, part_o, part_ml, nh, hd, out);
+    if (chunks == ATTN_CHUNKS)
+        hipLaunchKernelGGL(k_attention_merge<ATTN_CHUNKS>, dim3(nh), dim3(ATTN_CHUNKS * 8), 0, s, part_o, part_ml, nh, hd, out);
+    else
+        hipLaunchKernelGGL(k_attention_merge<ATTN_CHUNKS_LONG>, dim3(nh), dim3(ATTN_CHUNKS_LONG * 8), 0, s, part_o,
+                           part_ml, nh, hd, out);
     return hipGetLastError();
 }
 

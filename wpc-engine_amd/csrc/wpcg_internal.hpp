@@ -372,15 +372,18 @@ hipError_t launch_attention(int mode, const float* q, const float* k, const floa
 // merges them (XF_MERGE). Needs attention_fast_ok (head_dim 64 or 128).
 // rope: the step's RoPE row, cos then sin at the position (hd floats, as
 // launch_embed_tok leaves it); cache_pos: positions per head in kc / vc.
-constexpr int ATTN_CHUNKS = 16;
+//
+// chunks: ATTN_CHUNKS, or ATTN_CHUNKS_LONG (then part_o and part_ml hold
+// that many, and launch_attention_merge merges them).
+constexpr int ATTN_CHUNKS = 16, ATTN_CHUNKS_LONG = 64;
 bool attention_fast_ok(int nh, int nkv, int hd);
 hipError_t launch_attention_chunks(const float* q, const float* k, const float* v, const float* qn,
                                    const float* kn, int nh, int nkv, int hd, float eps, float scale,
                                    const float* rope, int cache_pos, const DecodeState* st, float* kc,
-                                   float* vc, float* part_o, float* part_ml, hipStream_t s);
+                                   float* vc, float* part_o, float* part_ml, int chunks, hipStream_t s);
 // The chunk states of launch_attention_chunks merged into out [nh][hd], as
 // the XF_MERGE transform merges them (hd <= 128).
-hipError_t launch_attention_merge(const float* part_o, const float* part_ml, int nh, int hd, float* out,
+hipError_t launch_attention_merge(const float* part_o, const float* part_ml, int nh, int hd, int chunks, float* out,
                                   hipStream_t s);
 hipError_t launch_add(float* x, const float* y, int n, hipStream_t s);
 // ---- batched prefill (decode.hip, gemv.hip, moe.hip, prefill.hip) ---------
