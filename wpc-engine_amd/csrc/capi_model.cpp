@@ -56,7 +56,15 @@ struct wpcg_model {
     float* final_norm = nullptr;
     float *cos_t = nullptr, *sin_t = nullptr;  // [max_pos][head_dim/2]
     float *kc = nullptr, *vc = nullptr;        // [layer][kv_head][max_pos][head_dim]
-    DecodeState* st = nullptr;
+    DecodeState* st = nullptr;                 // right behind the logits, so one copy takes both
+    // The host's copy of *st, current when no step is under way (every call
+    // ends with the stream drained); hst_ok is false after a failed call.
+    DecodeState hst{};
+    bool hst_ok = true;
+    // pinned: the logits with the state behind them as a step returns them,
+    // and the tokens as a call takes them (max_pos of them)
+    float* pin_out = nullptr;
+    uint32_t* pin_tok = nullptr;
     uint32_t* tokens = nullptr;                // [max_pos + 1]
     float *residual = nullptr, *normed = nullptr, *q = nullptr, *k = nullptr, *v = nullptr;
     float *attn = nullptr, *g = nullptr, *u = nullptr,
@@ -147,6 +155,53 @@ void free_model(wpcg_model* m)
     if (m->embed) wpcg_linear_destroy(m->embed);
     if (m->lm_head) wpcg_linear_destroy(m->lm_head);
     for (void* p : m->allocs) (void)hipFree(p);
+    if (m->pin_out) (void)hipHostFree(m->pin_out);
+    if (m->pin_tok) (void)hipHostFree(m->pin_tok);
+}
+
+// floats from the logits to the state behind them
+size_t st_off(const wpcg_model* m) { return ((size_t)m->cfg.vocab + 3) / 4 * 4; }
+
+// The decode state as of the last call, read back if that call failed.
+int host_state(wpcg_model* m)
+{
+    if (m->hst_ok) return WPCG_OK;
+    WPCG_HIP(hipStreamSynchronize(m->ctx->stream));
+    WPCG_HIP(hipMemcpy(&m->hst, m->st, sizeof m->hst, hipMemcpyDeviceToHost));
+    m->hst_ok = true;
+    return WPCG_OK;
+}
+
+// Queues st (the state's new value, also the host's) and n tokens for the
+// positions from st.pos on. A one-thread launch takes the state by value and
+// the tokens come from pinned memory, where each of up to five blocking
+// copies of a few bytes cost a call 10-20 us (256-token prompt, 2
+// Qwen3-30B-A3B-shaped layers: 551 -> 462 us a call).
+int put_state(wpcg_model* m, const DecodeState& st, const uint32_t* toks, uint32_t n)
+{
+    hipStream_t s = m->ctx->stream;
+    m->hst_ok = false;  // until the call ends well
+    if (n > 1) {
+        std::memcpy(m->pin_tok, toks, (size_t)n * 4);
+        WPCG_HIP(launch_copy_words(m->tokens + st.pos, m->pin_tok, n, s));
+    }
+    WPCG_HIP(launch_set_state(m->st, m->tokens, st, n == 1 ? toks : nullptr, s));
+    m->hst = st;
+    return WPCG_OK;
+}
+
+// The end of a call: the logits (if wanted) and the state to the host.
+int take_state(wpcg_model* m, float* logits)
+{
+    hipStream_t s = m->ctx->stream;
+    const size_t V = m->cfg.vocab, off = st_off(m), sw = sizeof(DecodeState) / 4;
+    const size_t from = logits ? 0 : off;
+    WPCG_HIP(launch_copy_words(m->pin_out + from, m->logits + from, (uint32_t)(off + sw - from), s));
+    WPCG_HIP(hipStreamSynchronize(s));
+    if (logits) std::memcpy(logits, m->pin_out, V * 4);
+    std::memcpy(&m->hst, m->pin_out + off, sizeof m->hst);
+    m->hst_ok = true;
+    return WPCG_OK;
 }
 
 // The logits head as the reference's loaders choose it: the dense decoder
@@ -563,9 +618,7 @@ int prefill_run(wpcg_model* m, uint32_t pos0, uint32_t n, uint32_t n_prompt)
         WPCG_HIP(launch_rms_norm(WPCG_MODE_FAST, xl, m->final_norm, (int)c.hidden, c.eps, m->normed, s));
         if (int rc = wpcg_linear_matvec(head, m->normed, m->logits, s)) return rc;
     }
-    WPCG_HIP(hipStreamSynchronize(s));
-    DecodeState st{pos0 + n - 1, n_prompt, c.max_pos, 0};
-    WPCG_HIP(hipMemcpy(m->st, &st, sizeof st, hipMemcpyHostToDevice));
+    if (int rc = put_state(m, DecodeState{pos0 + n - 1, n_prompt, c.max_pos, 0}, nullptr, 0)) return rc;
     WPCG_HIP(launch_argmax_next(m->logits, (int)c.vocab, m->st, m->tokens, s));
     return WPCG_OK;
 }
@@ -592,11 +645,8 @@ int verify_run(wpcg_model* m, uint32_t pos0, uint32_t n)
     const float* bs[1] = {head->bias};
     WPCG_HIP(launch_gemm_packed_rows(ms, bs, &P.vlogits, 1, P.xf, P.xsum, (int)n, nullptr, s));
     WPCG_HIP(launch_argmax_rows(P.vlogits, (int)c.vocab, (int)n, P.vids, s));
-    WPCG_HIP(hipStreamSynchronize(s));
-    uint32_t last = 0;
-    WPCG_HIP(hipMemcpy(&last, P.vids + (n - 1), 4, hipMemcpyDeviceToHost));
-    DecodeState st{pos0 + n, 0xffffffffu, c.max_pos, last};
-    WPCG_HIP(hipMemcpy(m->st, &st, sizeof st, hipMemcpyHostToDevice));
+    // (the state's last token stays the host's business: the caller has every argmax)
+    if (int rc = put_state(m, DecodeState{pos0 + n, 0xffffffffu, c.max_pos, 0}, nullptr, 0)) return rc;
     return WPCG_OK;
 }
 
@@ -712,7 +762,6 @@ int wpcg_model_create(wpcg_ctx* ctx, int scheme, const wpcg_model_config* cfg, w
     const size_t cache = (size_t)c.n_layers * kvd * c.max_pos * 4;
     dev((void**)&m->kc, cache);
     dev((void**)&m->vc, cache);
-    dev((void**)&m->st, sizeof(DecodeState));
     dev((void**)&m->tokens, ((size_t)c.max_pos + 1) * 4);
     dev((void**)&m->residual, c.hidden * 4u);
     dev((void**)&m->normed, c.hidden * 4u);
@@ -723,7 +772,8 @@ int wpcg_model_create(wpcg_ctx* ctx, int scheme, const wpcg_model_config* cfg, w
     dev((void**)&m->g, inter * 4);
     dev((void**)&m->u, inter * 4);
     dev((void**)&m->h, inter * 4);
-    dev((void**)&m->logits, (size_t)c.vocab * 4);
+    dev((void**)&m->logits, (st_off(m.get()) * 4) + sizeof(DecodeState));
+    m->st = reinterpret_cast<DecodeState*>(m->logits + st_off(m.get()));
     if (attention_fast_ok((int)c.n_heads, (int)c.n_kv_heads, (int)hd)) {
         dev((void**)&m->part_o, (size_t)ATTN_CHUNKS_LONG * qd * 4);
         dev((void**)&m->part_ml, (size_t)ATTN_CHUNKS_LONG * c.n_heads * 2 * 4);
@@ -731,6 +781,11 @@ int wpcg_model_create(wpcg_ctx* ctx, int scheme, const wpcg_model_config* cfg, w
         dev((void**)&m->amax, (size_t)(c.vocab + TILE_ROWS - 1) / TILE_ROWS * 8);
         dev((void**)&m->o2, (size_t)c.hidden * 4);
         dev((void**)&m->d2, (size_t)2 * c.hidden * 4);
+    }
+    if (rc == WPCG_OK) {
+        hipError_t e = hipHostMalloc((void**)&m->pin_out, st_off(m.get()) * 4 + sizeof(DecodeState));
+        if (e == hipSuccess) e = hipHostMalloc((void**)&m->pin_tok, (size_t)c.max_pos * 4);
+        if (e != hipSuccess) rc = hip_fail(e, "model staging");
     }
     if (rc == WPCG_OK) {
         // RoPE angles as rope.rs:29-33 computes them: f64 pow, sin, cos, cast to f32
@@ -746,6 +801,7 @@ int wpcg_model_create(wpcg_ctx* ctx, int scheme, const wpcg_model_config* cfg, w
         if (e == hipSuccess) e = hipMemcpy(m->sin_t, sn.data(), sn.size() * 4, hipMemcpyHostToDevice);
         DecodeState st{0, 0, c.max_pos, 0};
         if (e == hipSuccess) e = hipMemcpy(m->st, &st, sizeof st, hipMemcpyHostToDevice);
+        m->hst = st;
         if (e != hipSuccess) rc = hip_fail(e, "model tables");
     }
     if (rc != WPCG_OK) {
@@ -937,8 +993,8 @@ int wpcg_model_reset(wpcg_model* m)
 {
     if (!m) return fail(WPCG_E_ARG, "null model");
     if (int rc = check_ctx(m->ctx)) return rc;
-    DecodeState st{0, 0, m->cfg.max_pos, 0};
-    WPCG_HIP(hipMemcpy(m->st, &st, sizeof st, hipMemcpyHostToDevice));
+    if (int rc = put_state(m, DecodeState{0, 0, m->cfg.max_pos, 0}, nullptr, 0)) return rc;
+    m->hst_ok = true;
     return WPCG_OK;
 }
 
@@ -946,10 +1002,8 @@ int wpcg_model_position(wpcg_model* m, uint32_t* pos)
 {
     if (!m || !pos) return fail(WPCG_E_ARG, "null argument");
     if (int rc = check_ctx(m->ctx)) return rc;
-    DecodeState st;
-    WPCG_HIP(hipStreamSynchronize(m->ctx->stream));
-    WPCG_HIP(hipMemcpy(&st, m->st, sizeof st, hipMemcpyDeviceToHost));
-    *pos = st.pos;
+    if (int rc = host_state(m)) return rc;
+    *pos = m->hst.pos;
     return WPCG_OK;
 }
 
@@ -958,22 +1012,15 @@ int wpcg_model_forward_token(wpcg_model* m, uint32_t token, float* logits, uint3
     if (!m) return fail(WPCG_E_ARG, "null model");
     if (token >= m->cfg.vocab) return fail(WPCG_E_ARG, "token id out of range");
     if (int rc = ready(m)) return rc;
-    hipStream_t s = m->ctx->stream;
-    DecodeState st;
-    WPCG_HIP(hipStreamSynchronize(s));
-    WPCG_HIP(hipMemcpy(&st, m->st, sizeof st, hipMemcpyDeviceToHost));
+    if (int rc = host_state(m)) return rc;
+    DecodeState st = m->hst;
     if (st.pos >= m->cfg.max_pos) return fail(WPCG_E_ARG, "KV cache full (max_pos reached)");
     // every token comes from the host: keep the argmax out of tokens[]
     st.n_prompt = 0xffffffffu;
-    WPCG_HIP(hipMemcpy(m->st, &st, sizeof st, hipMemcpyHostToDevice));
-    WPCG_HIP(hipMemcpy(m->tokens + st.pos, &token, 4, hipMemcpyHostToDevice));
+    if (int rc = put_state(m, st, &token, 1)) return rc;
     if (int rc = run_step(m, st.pos)) return rc;
-    WPCG_HIP(hipStreamSynchronize(s));
-    if (logits) WPCG_HIP(hipMemcpy(logits, m->logits, (size_t)m->cfg.vocab * 4, hipMemcpyDeviceToHost));
-    if (argmax) {
-        WPCG_HIP(hipMemcpy(&st, m->st, sizeof st, hipMemcpyDeviceToHost));
-        *argmax = st.last;
-    }
+    if (int rc = take_state(m, logits)) return rc;
+    if (argmax) *argmax = m->hst.last;
     return WPCG_OK;
 }
 
@@ -1013,10 +1060,8 @@ int wpcg_model_generate(wpcg_model* m, const uint32_t* prompt, uint32_t n_prompt
         if (prompt[i] >= m->cfg.vocab) return fail(WPCG_E_ARG, "prompt token id out of range");
     if (int rc = ready(m)) return rc;
     hipStream_t s = m->ctx->stream;
-    WPCG_HIP(hipStreamSynchronize(s));
-    DecodeState st{0, n_prompt, m->cfg.max_pos, 0};
-    WPCG_HIP(hipMemcpy(m->st, &st, sizeof st, hipMemcpyHostToDevice));
-    WPCG_HIP(hipMemcpy(m->tokens, prompt, (size_t)n_prompt * 4, hipMemcpyHostToDevice));
+    if (int rc = host_state(m)) return rc;
+    if (int rc = put_state(m, DecodeState{0, n_prompt, m->cfg.max_pos, 0}, prompt, n_prompt)) return rc;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     WPCG_HIP(hipEventCreate(&e0));
     WPCG_HIP(hipEventCreate(&e1));
@@ -1048,7 +1093,9 @@ int wpcg_model_generate(wpcg_model* m, const uint32_t* prompt, uint32_t n_prompt
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (rc != WPCG_OK) return rc;
-    WPCG_HIP(hipMemcpy(out, m->tokens + n_prompt, (size_t)n_new * 4, hipMemcpyDeviceToHost));
+    WPCG_HIP(launch_copy_words(m->pin_tok, m->tokens + n_prompt, n_new, s));
+    if (int r2 = take_state(m, nullptr)) return r2;
+    std::memcpy(out, m->pin_tok, (size_t)n_new * 4);
     return WPCG_OK;
 }
 
@@ -1066,28 +1113,21 @@ int wpcg_model_prefill(wpcg_model* m, const uint32_t* tokens, uint32_t n, float*
     for (uint32_t i = 0; i < n; i++)
         if (tokens[i] >= m->cfg.vocab) return fail(WPCG_E_ARG, "token id out of range");
     if (int rc = ready(m)) return rc;
-    hipStream_t s = m->ctx->stream;
-    DecodeState st;
-    WPCG_HIP(hipStreamSynchronize(s));
-    WPCG_HIP(hipMemcpy(&st, m->st, sizeof st, hipMemcpyDeviceToHost));
+    if (int rc = host_state(m)) return rc;
+    DecodeState st = m->hst;
     if ((uint64_t)st.pos + n > m->cfg.max_pos) return fail(WPCG_E_ARG, "KV cache full (max_pos reached)");
-    WPCG_HIP(hipMemcpy(m->tokens + st.pos, tokens, (size_t)n * 4, hipMemcpyHostToDevice));
     // every token comes from the host: keep the argmax out of tokens[]
     const uint32_t pos0 = st.pos;
     st.n_prompt = 0xffffffffu;
+    if (int rc = put_state(m, st, tokens, n)) return rc;
     if (m->mode == WPCG_MODE_FAST && m->use_prefill && prefill_ok(m)) {
         if (int rc = prefill_run(m, pos0, n, st.n_prompt)) return rc;
     } else {
-        WPCG_HIP(hipMemcpy(m->st, &st, sizeof st, hipMemcpyHostToDevice));
         for (uint32_t i = 0; i < n; i++)
             if (int rc = run_step(m, pos0 + i)) return rc;
     }
-    WPCG_HIP(hipStreamSynchronize(s));
-    if (logits) WPCG_HIP(hipMemcpy(logits, m->logits, (size_t)m->cfg.vocab * 4, hipMemcpyDeviceToHost));
-    if (argmax) {
-        WPCG_HIP(hipMemcpy(&st, m->st, sizeof st, hipMemcpyDeviceToHost));
-        *argmax = st.last;
-    }
+    if (int rc = take_state(m, logits)) return rc;
+    if (argmax) *argmax = m->hst.last;
     return WPCG_OK;
 }
 
@@ -1100,28 +1140,29 @@ int wpcg_model_verify(wpcg_model* m, const uint32_t* tokens, uint32_t n, uint32_
     if (int rc = ready(m)) return rc;
     hipStream_t s = m->ctx->stream;
     const size_t V = m->cfg.vocab;
-    DecodeState st;
-    WPCG_HIP(hipStreamSynchronize(s));
-    WPCG_HIP(hipMemcpy(&st, m->st, sizeof st, hipMemcpyDeviceToHost));
+    if (int rc = host_state(m)) return rc;
+    DecodeState st = m->hst;
     if ((uint64_t)st.pos + n > m->cfg.max_pos) return fail(WPCG_E_ARG, "KV cache full (max_pos reached)");
-    WPCG_HIP(hipMemcpy(m->tokens + st.pos, tokens, (size_t)n * 4, hipMemcpyHostToDevice));
     const uint32_t pos0 = st.pos;
+    st.n_prompt = 0xffffffffu;
+    if (int rc = put_state(m, st, tokens, n)) return rc;
     if (m->mode == WPCG_MODE_FAST && m->use_prefill && prefill_ok(m)) {
         if (int rc = verify_run(m, pos0, n)) return rc;
-        WPCG_HIP(hipMemcpy(argmax, m->pf.vids, (size_t)n * 4, hipMemcpyDeviceToHost));
+        WPCG_HIP(launch_copy_words(m->pin_tok, m->pf.vids, n, s));
+        WPCG_HIP(hipStreamSynchronize(s));
+        std::memcpy(argmax, m->pin_tok, (size_t)n * 4);
         if (logits) WPCG_HIP(hipMemcpy(logits, m->pf.vlogits, (size_t)n * V * 4, hipMemcpyDeviceToHost));
+        m->hst_ok = true;
         return WPCG_OK;
     }
     // step by step (EXACT: the reference's steps exactly)
-    st.n_prompt = 0xffffffffu;
-    WPCG_HIP(hipMemcpy(m->st, &st, sizeof st, hipMemcpyHostToDevice));
     for (uint32_t i = 0; i < n; i++) {
         if (int rc = run_step(m, pos0 + i)) return rc;
-        WPCG_HIP(hipStreamSynchronize(s));
-        if (logits) WPCG_HIP(hipMemcpy(logits + i * V, m->logits, V * 4, hipMemcpyDeviceToHost));
-        WPCG_HIP(hipMemcpy(&st, m->st, sizeof st, hipMemcpyDeviceToHost));
-        argmax[i] = st.last;
+        if (int rc = take_state(m, logits ? logits + i * V : nullptr)) return rc;
+        m->hst_ok = false;
+        argmax[i] = m->hst.last;
     }
+    m->hst_ok = true;
     return WPCG_OK;
 }
 
@@ -1129,12 +1170,12 @@ int wpcg_model_set_position(wpcg_model* m, uint32_t pos)
 {
     if (!m) return fail(WPCG_E_ARG, "null model");
     if (int rc = check_ctx(m->ctx)) return rc;
-    DecodeState st;
-    WPCG_HIP(hipStreamSynchronize(m->ctx->stream));
-    WPCG_HIP(hipMemcpy(&st, m->st, sizeof st, hipMemcpyDeviceToHost));
+    if (int rc = host_state(m)) return rc;
+    DecodeState st = m->hst;
     if (pos > st.pos) return fail(WPCG_E_ARG, "set_position only moves back (to drop rejected tokens)");
     st.pos = pos;
-    WPCG_HIP(hipMemcpy(m->st, &st, sizeof st, hipMemcpyHostToDevice));
+    if (int rc = put_state(m, st, nullptr, 0)) return rc;
+    m->hst_ok = true;
     return WPCG_OK;
 }
 

@@ -1152,6 +1152,22 @@ __global__ __launch_bounds__(NCH * 8) void k_attention_merge(const float* __rest
     if (on) out[(size_t)h * hd + d] = a * __fdiv_rn(1.0f, L);
 }
 
+// ---- between the host and the decode's buffers -----------------------------
+__global__ void k_set_state(DecodeState* st, uint32_t* tokens, DecodeState v, uint32_t tok, int put)
+{
+    *st = v;
+    if (put) tokens[v.pos] = tok;
+}
+
+// Pinned host memory is written and read straight from the kernel (a copy
+// engine's hand-over costs more than the few hundred KB of a step's logits).
+__global__ __launch_bounds__(256) void k_copy_words(uint32_t* __restrict__ dst, const uint32_t* __restrict__ src,
+                                                    uint32_t n)
+{
+    for (uint32_t i = blockIdx.x * 1024 + threadIdx.x, k = 0; k < 4; k++, i += 256)
+        if (i < n) dst[i] = src[i];
+}
+
 // ---- argmax (sampling.rs:3-14) and the next step's input -------------------
 // First index of the largest logit (strict >, so NaN never wins; 0 when no
 // logit beats -inf).
@@ -1463,6 +1479,22 @@ hipError_t launch_attention_merge(const float* part_o, const float* part_ml, int
     else
         hipLaunchKernelGGL(k_attention_merge<ATTN_CHUNKS_LONG>, dim3(nh), dim3(ATTN_CHUNKS_LONG * 8), 0, s, part_o,
                            part_ml, nh, hd, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_set_state(DecodeState* st, uint32_t* tokens, const DecodeState& v, const uint32_t* tok, hipStream_t s)
+{
+    (void)hipGetLastError();
+    hipLaunchKernelGGL(k_set_state, dim3(1), dim3(1), 0, s, st, tokens, v, tok ? *tok : 0u, tok ? 1 : 0);
+    return hipGetLastError();
+}
+
+hipError_t launch_copy_words(void* dst, const void* src, uint32_t n, hipStream_t s)
+{
+    if (!n) return hipSuccess;
+    (void)hipGetLastError();
+    hipLaunchKernelGGL(k_copy_words, dim3((n + 1023) / 1024), dim3(256), 0, s, static_cast<uint32_t*>(dst),
+                       static_cast<const uint32_t*>(src), n);
     return hipGetLastError();
 }
 

@@ -386,6 +386,10 @@ hipError_t launch_attention_chunks(const float* q, const float* k, const float* 
 hipError_t launch_attention_merge(const float* part_o, const float* part_ml, int nh, int hd, int chunks, float* out,
                                   hipStream_t s);
 hipError_t launch_add(float* x, const float* y, int n, hipStream_t s);
+// *st = v, and tokens[v.pos] = *tok if tok (host) is set.
+hipError_t launch_set_state(DecodeState* st, uint32_t* tokens, const DecodeState& v, const uint32_t* tok, hipStream_t s);
+// n words from src to dst, either of them pinned host memory.
+hipError_t launch_copy_words(void* dst, const void* src, uint32_t n, hipStream_t s);
 // ---- batched prefill (decode.hip, gemv.hip, moe.hip, prefill.hip) ---------
 // n tokens at positions pos0 .. pos0+n-1, row t of every batch buffer being
 // position pos0 + t.
