@@ -173,6 +173,28 @@ def test_fast_prefill_v3_matches_steps(ctx, name, cfg, n, seed):
     m.close()
 
 
+@pytest.mark.parametrize("n", [2, 15, 16, 17, 33, 1024, 1041])
+def test_fast_dense_prefill_rows(ctx, n):
+    """The dense pass at the edges of its 16- and 32-row tiles and of a pass
+    (1024 rows, then 1024 + 17), an odd number of 128-value blocks in the down
+    projection (whose packed input the SiLU writes), against the FAST steps of
+    the same model: TOL as above."""
+    cfg = dict(DENSE, n_heads=2, n_kv_heads=1, head_dim=128, inter=640, max_pos=1088)
+    print(f"[gpu] dense prefill of {n} rows", flush=True)
+    m = build(ctx, cfg, 61, wpcg.MODE_FAST)
+    toks = np.random.default_rng(n).integers(0, cfg["vocab"], n).astype(np.uint32)
+    for t in toks:
+        ref, ref_id = m.forward_token(int(t))
+    kr, vr = cache(m, cfg, n)
+    m.reset()
+    got, got_id = m.prefill(toks)
+    kg, vg = cache(m, cfg, n)
+    assert float(np.max(np.abs(got - ref))) <= TOL * float(ref.max() - ref.min()) and got_id == ref_id
+    assert float(np.max(np.abs(kg - kr))) <= TOL * float(np.max(np.abs(kr)))
+    assert float(np.max(np.abs(vg - vr))) <= TOL * float(np.max(np.abs(vr)))
+    m.close()
+
+
 def test_exact_prefill_is_the_steps(ctx):
     cfg = MOE
     m = build(ctx, cfg, 41, wpcg.MODE_EXACT)

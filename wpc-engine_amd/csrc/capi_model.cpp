@@ -563,8 +563,7 @@ int prefill_pass(wpcg_model* m, uint32_t pos0, uint32_t n, hipStream_t s)
             const float* bs[2] = {L.gate->bias, L.up->bias};
             float* ys[2] = {P.g, P.u};
             WPCG_HIP(launch_gemm_packed_rows(ms, bs, ys, 2, P.xf, P.xsum, (int)n, nullptr, s));
-            WPCG_HIP(launch_silu_mul(P.g, P.u, P.g, (size_t)n * c.inter, s));
-            WPCG_HIP(launch_gemm_pack_rows(P.g, (int)n, (int)c.inter, P.xf, P.xsum, s));
+            WPCG_HIP(launch_silu_pack_rows(P.g, P.u, (int)n, (int)c.inter, P.xf, P.xsum, s));
             WPCG_HIP(residual(L.down));
             continue;
         }

@@ -413,6 +413,8 @@ hipError_t launch_route_rows(const float* scores, int n, int rows, int top_k, in
 // launch_gemm_pack_rows's layout), H % 128 == 0.
 hipError_t launch_rms_pack_rows(const float* X, const float* w, int n, int H, float eps, void* xf, float* xsum,
                                 hipStream_t s);
+// silu(G) * U (n rows of K, K % 128 == 0) into the same layout.
+hipError_t launch_silu_pack_rows(const float* G, const float* U, int n, int K, void* xf, float* xsum, hipStream_t s);
 // Each row's FAST RMSNorm with weights w of X [M][H] into XN; H <=
 // PF_NORM_MAXH. dg non-null: XN's rows also as launch_pf_digits writes them
 // (dg, dxs), H % 128 == 0.
