@@ -173,14 +173,16 @@ def test_fast_prefill_v3_matches_steps(ctx, name, cfg, n, seed):
     m.close()
 
 
-@pytest.mark.parametrize("n", [2, 15, 16, 17, 33, 1024, 1041])
-def test_fast_dense_prefill_rows(ctx, n):
+@pytest.mark.parametrize("n,hidden", [(2, 256), (15, 256), (16, 256), (17, 256), (33, 256), (1024, 256), (1041, 256),
+                                      (830, 2688)])
+def test_fast_dense_prefill_rows(ctx, n, hidden):
     """The dense pass at the edges of its 16- and 32-row tiles and of a pass
     (1024 rows, then 1024 + 17), an odd number of 128-value blocks in the down
-    projection (whose packed input the SiLU writes), against the FAST steps of
-    the same model: TOL as above."""
-    cfg = dict(DENSE, n_heads=2, n_kv_heads=1, head_dim=128, inter=640, max_pos=1088)
-    print(f"[gpu] dense prefill of {n} rows", flush=True)
+    projection (whose packed input the SiLU writes), and rows and blocks enough
+    for the norm's workgroups to take two blocks each, an odd count of them,
+    against the FAST steps of the same model: TOL as above."""
+    cfg = dict(DENSE, hidden=hidden, n_heads=2, n_kv_heads=1, head_dim=128, inter=640, max_pos=1088)
+    print(f"[gpu] dense prefill of {n} rows of {hidden}", flush=True)
     m = build(ctx, cfg, 61, wpcg.MODE_FAST)
     toks = np.random.default_rng(n).integers(0, cfg["vocab"], n).astype(np.uint32)
     for t in toks:

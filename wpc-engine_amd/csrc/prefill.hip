@@ -7,6 +7,8 @@
 //   expert loop, combine  qwen3_moe_model.rs:509-530
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #define REF_EXPF_FN __device__ __forceinline__
 #include "ref_expf.h"
 #include "wave.h"
@@ -95,18 +97,24 @@ __global__ __launch_bounds__(RT_WG) void k_pf_router(const float* __restrict__ X
 // 1 / sqrt(mean + eps), then (x * scale) * w) written straight as the
 // GEMM's packed X, with no fp32 copy and no packing launch: workgroup
 // (16-row tile q, block b). Every workgroup of a tile computes its 16 row
-// norms itself (each row is read from L2 once per block: 256 workgroups for
-// 256 rows of 2048 beat 64 workgroups of four blocks each, 15 us), then
-// stages its block of the normed rows in LDS and packs it.
-constexpr int RP_BG = 1;
+// norms itself, then stages its blocks of the normed rows in LDS, one after
+// another, and packs them. Bound by reading the rows again for the norms:
+// the workgroups of a tile share an XCD, so that its L2 serves them
+// (1000 rows of 2560: spread over all eight L2s 30 us, now 10.4), and take bg
+// blocks each once there are more than 512 of them (256 rows of 2048: 256
+// workgroups of one block 5.5 us, 64 of four 15).
 __global__ __launch_bounds__(256) void k_rms_pack(const float* __restrict__ X, const float* __restrict__ w, int n,
-                                                  int H, float eps, int XT, uint32_t* __restrict__ xf,
+                                                  int H, float eps, int bg, int XT, uint32_t* __restrict__ xf,
                                                   float* __restrict__ xsum)
 {
     __shared__ float rstd[16];
     __shared__ __align__(16) float tile[16][132];
     __shared__ float red[2][4][16];
-    const int q = blockIdx.x, r = threadIdx.x >> 4, p = threadIdx.x & 15;
+    // XCD x (workgroups x, x + 8, ...) takes tiles x, x + 8, ...
+    const int groups = (H / 128 + bg - 1) / bg, i = (int)blockIdx.x >> 3;
+    const int q = ((int)blockIdx.x & 7) + 8 * (i / groups), b0 = i % groups * bg;
+    if (16 * q >= n) return;
+    const int r = threadIdx.x >> 4, p = threadIdx.x & 15;
     const int row = 16 * q + r;
     // row r's squares by its 16 threads (lanes 16r..16r+15 of one wave)
     float ss = 0.0f;
@@ -125,9 +133,9 @@ __global__ __launch_bounds__(256) void k_rms_pack(const float* __restrict__ X, c
     ss += __shfl_xor(ss, 1);
     if (p == 0) rstd[r] = __fdiv_rn(1.0f, __builtin_sqrtf(__fadd_rn(__fdiv_rn(ss, (float)H), eps)));
     __syncthreads();
-    const int b1 = min(H / 128, (int)(blockIdx.y + 1) * RP_BG);
+    const int b1 = min(H / 128, b0 + bg);
     const int rr = threadIdx.x >> 4, cc = (threadIdx.x & 15) * 8, mrow = 16 * q + rr;
-    for (int b = blockIdx.y * RP_BG; b < b1; b++) {
+    for (int b = b0; b < b1; b++) {
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             const int k = b * 128 + cc + 4 * h;
@@ -358,8 +366,10 @@ hipError_t launch_rms_pack_rows(const float* X, const float* w, int n, int H, fl
 {
     if (n < 1 || H < 128 || H % 128) return hipErrorInvalidValue;
     (void)hipGetLastError();
-    const dim3 grid((unsigned)((n + 15) / 16), (unsigned)((H / 128 + RP_BG - 1) / RP_BG));
-    hipLaunchKernelGGL(k_rms_pack, grid, dim3(256), 0, s, X, w, n, H, eps, gemm_rows_tiles(n),
+    const int nb = H / 128, tiles = (n + 15) / 16;
+    const int bg = std::max(1, (int)((int64_t)tiles * nb / 512));
+    const unsigned grid = (unsigned)((tiles + 7) / 8 * 8 * ((nb + bg - 1) / bg));
+    hipLaunchKernelGGL(k_rms_pack, dim3(grid), dim3(256), 0, s, X, w, n, H, eps, bg, gemm_rows_tiles(n),
                        static_cast<uint32_t*>(xf), xsum);
     return hipGetLastError();
 }
