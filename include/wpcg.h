@@ -410,7 +410,10 @@ int wpcg_model_set_mode(wpcg_model* m, int mode);
  * by launch (for tools that cannot trace graph replays). No reference
  * counterpart. */
 int wpcg_model_set_graphs(wpcg_model* m, int enabled);
-/* Empty the KV cache (position 0). */
+/* Empty the KV cache (position 0). Like wpcg_model_set_position it returns
+ * with the new position queued on the context's stream; later calls on the
+ * model see it at once. No call on a model can be made while the context's
+ * stream is being captured (wpcg_graph_begin): E_ARG. */
 int wpcg_model_reset(wpcg_model* m);
 int wpcg_model_position(wpcg_model* m, uint32_t* pos);
 /* One step at the next position with input `token`: logits (host, vocab

@@ -304,3 +304,33 @@ def test_model_loads_from_checkpoint(ctx, tmp_path, name, cfg, scheme, dtype, sh
     print(f"[gpu] checkpoint load {name}: 12 steps bit-identical", flush=True)
     m.close()
     ref.close()
+
+
+def test_model_calls_are_refused_while_the_stream_is_captured(ctx):
+    """A recorded reset or set_position would move the host's idea of the
+    position and leave the device's where it was."""
+    m, ref = build(ctx, DENSE, 21)
+    ref.close()
+    m.set_mode(wpcg.MODE_FAST)
+    a = m.prefill(np.arange(5, dtype=np.uint32))[0]
+    lin = wpcg.WpcLinear.from_blocks(ctx, 4, synth.random_v4_blocks(64, 256, 1), 64, 256)
+    x, y = ctx.upload(synth.random_x(256, seed=2)), ctx.alloc(4 * 64)
+    calls = [m.reset, lambda: m.set_position(2), m.position, lambda: m.forward_token(1),
+             lambda: m.prefill(np.arange(3, dtype=np.uint32)), lambda: m.verify(np.arange(3, dtype=np.uint32)),
+             lambda: m.generate(np.arange(3, dtype=np.uint32), 2)]
+
+    def captured():
+        lin.matvec_dev(x, y)
+        for call in calls:
+            with pytest.raises(wpcg.WpcgError):
+                call()
+
+    g = ctx.capture(captured)  # the graph itself is whole
+    g.launch()
+    ctx.sync()
+    assert m.position() == 5
+    m.set_position(0)
+    assert np.array_equal(m.prefill(np.arange(5, dtype=np.uint32))[0], a)
+    del g
+    lin.close()
+    m.close()

@@ -57,8 +57,10 @@ struct wpcg_model {
     float *cos_t = nullptr, *sin_t = nullptr;  // [max_pos][head_dim/2]
     float *kc = nullptr, *vc = nullptr;        // [layer][kv_head][max_pos][head_dim]
     DecodeState* st = nullptr;                 // right behind the logits, so one copy takes both
-    // The host's copy of *st, current when no step is under way (every call
-    // ends with the stream drained); hst_ok is false after a failed call.
+    // The host's copy of *st, current whenever no call is under way: calls
+    // that run steps end with the stream drained, reset and set_position only
+    // queue the value that the copy already has (later calls are queued behind
+    // it). hst_ok is false after a failed call.
     DecodeState hst{};
     bool hst_ok = true;
     // pinned: the logits with the state behind them as a step returns them,
@@ -157,6 +159,18 @@ void free_model(wpcg_model* m)
     for (void* p : m->allocs) (void)hipFree(p);
     if (m->pin_out) (void)hipHostFree(m->pin_out);
     if (m->pin_tok) (void)hipHostFree(m->pin_tok);
+}
+
+// Every call on a model waits for the stream or queues work that later calls
+// rely on, so none can be recorded into a graph (a recorded reset would leave
+// the device's state as it was).
+int not_capturing(wpcg_model* m)
+{
+    if (int rc = check_ctx(m->ctx)) return rc;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    WPCG_HIP(hipStreamIsCapturing(m->ctx->stream, &st));
+    if (st != hipStreamCaptureStatusNone) return fail(WPCG_E_ARG, "model call while the context's stream is captured");
+    return WPCG_OK;
 }
 
 // floats from the logits to the state behind them
@@ -693,7 +707,7 @@ int ready(wpcg_model* m)
 {
     const std::string miss = missing(m);
     if (!miss.empty()) return fail(WPCG_E_ARG, "tensor not set: " + miss);
-    return check_ctx(m->ctx);
+    return not_capturing(m);
 }
 
 }  // namespace
@@ -991,7 +1005,7 @@ int wpcg_model_set_graphs(wpcg_model* m, int enabled)
 int wpcg_model_reset(wpcg_model* m)
 {
     if (!m) return fail(WPCG_E_ARG, "null model");
-    if (int rc = check_ctx(m->ctx)) return rc;
+    if (int rc = not_capturing(m)) return rc;
     // (after a failed call: what it left queued may still read the pinned tokens)
     if (!m->hst_ok) WPCG_HIP(hipStreamSynchronize(m->ctx->stream));
     if (int rc = put_state(m, DecodeState{0, 0, m->cfg.max_pos, 0}, nullptr, 0)) return rc;
@@ -1002,7 +1016,7 @@ int wpcg_model_reset(wpcg_model* m)
 int wpcg_model_position(wpcg_model* m, uint32_t* pos)
 {
     if (!m || !pos) return fail(WPCG_E_ARG, "null argument");
-    if (int rc = check_ctx(m->ctx)) return rc;
+    if (int rc = not_capturing(m)) return rc;
     if (int rc = host_state(m)) return rc;
     *pos = m->hst.pos;
     return WPCG_OK;
@@ -1176,7 +1190,7 @@ int wpcg_model_verify(wpcg_model* m, const uint32_t* tokens, uint32_t n, uint32_
 int wpcg_model_set_position(wpcg_model* m, uint32_t pos)
 {
     if (!m) return fail(WPCG_E_ARG, "null model");
-    if (int rc = check_ctx(m->ctx)) return rc;
+    if (int rc = not_capturing(m)) return rc;
     if (int rc = host_state(m)) return rc;
     DecodeState st = m->hst;
     if (pos > st.pos) return fail(WPCG_E_ARG, "set_position only moves back (to drop rejected tokens)");
