@@ -14,8 +14,8 @@ void free_gemm(GemmWork& w)
     if (w.xsum) (void)hipFree(w.xsum);
     if (w.part) (void)hipFree(w.part);
     if (w.counters) (void)hipFree(w.counters);
-    if (w.wxf) (void)hipFree(w.wxf);
-    if (w.wxsum) (void)hipFree(w.wxsum);
+    for (void* p : w.wide)
+        if (p) (void)hipFree(p);
     const int req = w.kg_req;
     w = GemmWork{};
     w.kg_req = req;
@@ -56,30 +56,37 @@ bool wide(const wpcg_linear* L, int x_mode, uint32_t M)
            L->m.nb * GEMM_WIDE_TILES * 4096 < (1ull << 30);  // the kernel's buffer offsets
 }
 
-// The many-row kernel over M rows. Its packed X is allocated by the first
-// such call; while a graph is being captured (no allocation) the 64-column
-// workspace serves in smaller passes, with the same results.
+// The many-row kernel over M rows. Its packed X is made by the first call
+// that wants its size (the least of 8, 16, ... GEMM_WIDE_TILES tiles that
+// hold the rows, so at most twice what the largest call needs stays held).
+// While a graph is being captured, or where the memory is not there, the
+// largest one made, or the 64-column workspace, serves in smaller passes,
+// with the same results.
 int run_wide(wpcg_linear* L, const void* x, int x_mode, uint32_t M, const float* res, float* y, hipStream_t s)
 {
     const DeviceMatrix& m = L->m;
     GemmWork& w = L->gemm;
-    if (!w.wxf) {
+    constexpr int N = sizeof w.wide / sizeof w.wide[0];
+    static_assert((8 << (N - 1)) == GEMM_WIDE_TILES, "the steps end at a whole pass");
+    int want = 0;
+    while (want < N - 1 && (uint32_t)gemm_wide_cols(x_mode, gemm_wide_step(want)) < M) want++;
+    int i = want;
+    while (i < N && !w.wide[i]) i++;
+    if (i == N) {
+        i = want;
         hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
         WPCG_HIP(hipStreamIsCapturing(s, &st));
-        if (st != hipStreamCaptureStatusNone) {
-            WPCG_HIP(launch_gemm_wide(m, w.xf, w.xsum, GEMM_MAX_M / 16, x, x_mode, M, L->bias, res, y, s));
-            return WPCG_OK;
+        if (st == hipStreamCaptureStatusNone &&
+            hipMalloc(&w.wide[i], m.nb * gemm_wide_step(i) * (4096 + 16 * sizeof(float))) != hipSuccess) {
+            (void)hipGetLastError();
+            w.wide[i] = nullptr;
         }
-        void* f = nullptr;
-        hipError_t e = hipMalloc(&f, m.nb * GEMM_WIDE_TILES * 4096);
-        if (e == hipSuccess) e = hipMalloc(&w.wxsum, m.nb * GEMM_WIDE_TILES * 16 * sizeof(float));
-        if (e != hipSuccess) {
-            if (f) (void)hipFree(f);
-            return hip_fail(e, "batched GEMM workspace");
-        }
-        w.wxf = f;
+        while (i >= 0 && !w.wide[i]) i--;
     }
-    WPCG_HIP(launch_gemm_wide(m, w.wxf, w.wxsum, GEMM_WIDE_TILES, x, x_mode, M, L->bias, res, y, s));
+    const int tiles = i < 0 ? GEMM_MAX_M / 16 : gemm_wide_step(i);
+    void* xf = i < 0 ? w.xf : w.wide[i];
+    float* xsum = i < 0 ? w.xsum : reinterpret_cast<float*>(static_cast<uint8_t*>(xf) + m.nb * tiles * 4096);
+    WPCG_HIP(launch_gemm_wide(m, xf, xsum, tiles, x, x_mode, M, L->bias, res, y, s));
     return WPCG_OK;
 }
 

@@ -201,6 +201,8 @@ constexpr int GEMM_WG_THREADS = 512;
 constexpr int GEMM_TILES_PER_WAVE = 1;
 constexpr int GEMM_MAX_M = 64;
 constexpr int GEMM_SMALL_MAXBK = 30;
+constexpr int GEMM_WIDE_TILES = 128;                 // 16-column tiles of packed X in a pass of gemm_wide.hip
+inline int gemm_wide_step(int i) { return 8 << i; }  // the sizes of its workspace, up to that
 // Workspace of one matrix, sized for GEMM_MAX_M columns; fixed once made so
 // captured graphs keep valid pointers.
 struct GemmWork {
@@ -211,8 +213,10 @@ struct GemmWork {
     float* xsum = nullptr;          // per-block column sums: nb * 64
     float* part = nullptr;          // partial Y: [kg][64][rows_pad] or [kg_small][16][rows_pad]
     uint32_t* counters = nullptr;   // one per row group, self-resetting
-    void* wxf = nullptr;            // the many-row kernel's packed X: nb * GEMM_WIDE_TILES tiles * 4 KiB
-    float* wxsum = nullptr;         // its column sums: nb * GEMM_WIDE_TILES * 16
+    // the many-row kernel's packed X, [i] of gemm_wide_step(i) column tiles:
+    // nb * tiles * 4 KiB, then nb * tiles * 16 column sums. Each is made by
+    // the first call that wants its size and kept (captured graphs).
+    void* wide[5] = {};
 };
 void free_gemm(GemmWork& w);  // keeps kg_req
 int gemm_row_groups(uint64_t rows);        // more than 16 columns
@@ -232,7 +236,7 @@ hipError_t launch_gemm(const DeviceMatrix& m, const GemmWork& w, const void* x, 
 // passes of gemm_wide_cols(x_mode, tiles) rows into `tiles` 16-column tiles
 // of xf / xsum, then one launch covers every row of the pass. An output
 // does not depend on the passes it is split into.
-constexpr int GEMM_WIDE_TILES = 128;  // 2048 rows of X a pass, 1024 in the SPLIT mode
+// GEMM_WIDE_TILES hold 2048 rows of X a pass, 1024 in the SPLIT mode.
 inline int gemm_wide_cols(int x_mode, int tiles) { return x_mode == GX_SPLIT ? tiles / 4 * 32 : tiles / 2 * 32; }
 hipError_t launch_gemm_wide(const DeviceMatrix& m, void* xf, float* xsum, int tiles, const void* x, int x_mode,
                             uint32_t M, const float* bias, const float* res, float* y, hipStream_t s);
