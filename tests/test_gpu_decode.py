@@ -48,6 +48,9 @@ QWEN3_4B_2L = dict(n_layers=2, hidden=2560, n_heads=32, n_kv_heads=8, head_dim=1
 ODD_OPROJ = dict(n_layers=2, hidden=256, n_heads=6, n_kv_heads=2, head_dim=64, inter=384, vocab=1000,
                  n_experts=0, top_k=0, moe_inter=0, norm_topk=1, tied=1, max_pos=96, eps=1e-6,
                  rope_theta=1e6)
+# The down projection's 97 blocks are four K-slices, which join inside its
+# launch: the residual's deferred o_proj slice has to be added there
+FOUR_SLICE_DOWN = dict(DENSE, inter=128 * 97)
 # Long contexts: past 16 x 32 = 512 positions each FAST attention chunk holds
 # a second block of 32 positions, past 1024 a third. LONG: head_dim 64 with
 # 2 query heads per key head (the 512-thread attention); LONG_REP8: head_dim
@@ -138,6 +141,7 @@ def test_exact_decode_is_bit_identical(ctx, name, cfg, n_prompt, n_new, seed):
                                                     ("qwen3-moe-2L", QWEN3_MOE_2L, 78, 313),
                                                     ("qwen3-4b-2L", QWEN3_4B_2L, 90, 414),
                                                     ("odd-oproj", ODD_OPROJ, 90, 515),
+                                                    ("four-slice-down", FOUR_SLICE_DOWN, 20, 919),
                                                     ("long", LONG, 1060, 616),
                                                     ("long-rep8", LONG_REP8, 1060, 717)])
 def test_fast_decode_tracks_the_reference(ctx, name, cfg, n_steps, seed):

@@ -1075,18 +1075,21 @@ __global__ __launch_bounds__(FAST_WG, KIND == FK_PLAIN && (XF == XF_NONE || (XF 
         for (int k = 1; k < kw; k++) sum += red[tt * kw + k][rr];
         if constexpr (xform == XF_NORM) sum *= rscale;
     }
+    // v plus the row's bias and deferred slices
+    auto biased = [&](float v) {
+        if (!out_bias) return v;
+        float b = out_bias[orow];
+        if (out_bias2) {
+            b += out_bias2[orow];
+            if (out_nb2 > 1) b += out_bias2[(size_t)out_rows + orow];
+        }
+        return v + b;
+    };
     if (kg == 1 || out_y2) {  // one slice, or the deferred split: slices k >= 1 to y2
         const bool row_ok = mine && orow < (size_t)out_rows;
         if (row_ok) {
             if (kgi == 0) {
-                if (out_bias) {
-                    float b = out_bias[orow];
-                    if (out_bias2) {
-                        b += out_bias2[orow];
-                        if (out_nb2 > 1) b += out_bias2[(size_t)out_rows + orow];
-                    }
-                    sum += b;
-                }
+                sum = biased(sum);
                 out_y[orow] = sum;
             } else {
                 out_y2[(size_t)(kgi - 1) * out_rows + orow] = sum;
@@ -1143,7 +1146,7 @@ __global__ __launch_bounds__(FAST_WG, KIND == FK_PLAIN && (XF == XF_NONE || (XF 
         for (int k = 1; k < kg; k++)
             acc += __hip_atomic_load(P.part + (size_t)k * P.rows_pad + orow, __ATOMIC_RELAXED,
                                      __HIP_MEMORY_SCOPE_AGENT);
-        out_y[orow] = out_bias ? acc + out_bias[orow] : acc;
+        out_y[orow] = biased(acc);
     }
     if (t == 0) __hip_atomic_store(P.counters + tg, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
