@@ -426,7 +426,8 @@ int wpcg_model_forward_token(wpcg_model* m, uint32_t token, float* logits, uint3
  * prompt token, keeping the last logits) for n tokens at the next n
  * positions: the same result as n forward_token calls, logits and argmax of
  * the last. EXACT mode runs exactly those steps (bit-identical). FAST mode
- * runs the tokens as batches of up to 256 rows (the reference's missing
+ * runs the tokens as batches of up to 256 rows (dense models: up to 1024,
+ * made when a prompt of more than 256 comes; the reference's missing
  * batched prefill, README.md:174-180): every layer reads each weight once
  * per batch; the dense projections run on the matrix cores with X carried
  * as two bf16 terms (WPCG_DTYPE_F32_SPLIT), attention is causal over the

@@ -1,7 +1,8 @@
 // The workspace rules of the batched GEMM (csrc/capi_gemm.cpp) with the HIP
 // calls and kernel launchers replaced by counters: how much a call allocates,
 // what it falls back to when an allocation fails or a graph is captured, and
-// that what a captured graph may hold stays allocated.
+// that what a captured graph may hold stays allocated. Then the rows of the
+// prefill's batch buffers (grow_rows).
 #include "../../wpc-engine_amd/csrc/capi_gemm.cpp"
 
 #include <cstdio>
@@ -163,6 +164,26 @@ int main()
         CHECK(gemm(L, bf, 130) == WPCG_OK && launched.empty() && passes == 3);
         CHECK(gemm(L, sp, 70) == WPCG_OK && launched.empty() && passes == 6);
         free_gemm(L.gemm);
+    }
+    {  // the prefill's rows: as many as wanted, else those there, else the least
+        uint32_t have = 0, most = 1024;
+        std::vector<uint32_t> asked;
+        auto make = [&](uint32_t rows) {
+            asked.push_back(rows);
+            if (rows > most) return WPCG_E_DEVICE;
+            have = rows;
+            return WPCG_OK;
+        };
+        CHECK(grow_rows(have, 256, 256, make) == WPCG_OK && have == 256);
+        CHECK(grow_rows(have, 256, 256, make) == WPCG_OK && asked.size() == 1);
+        most = 500;
+        CHECK(grow_rows(have, 1024, 256, make) == WPCG_OK && have == 256 && asked.size() == 2);
+        most = 1024;
+        CHECK(grow_rows(have, 1024, 256, make) == WPCG_OK && have == 1024);
+        have = 0, most = 300;
+        CHECK(grow_rows(have, 1024, 256, make) == WPCG_OK && have == 256);
+        have = 0, most = 100;
+        CHECK(grow_rows(have, 1024, 256, make) != WPCG_OK && grow_rows(have, 256, 256, make) != WPCG_OK && have == 0);
     }
     std::printf("workspace ok\n");
     return 0;

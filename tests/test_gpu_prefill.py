@@ -17,6 +17,8 @@ Speculative verification is held to the same bars against the oracle's
 steps. Cases cover one pass, several passes (more tokens than a pass holds),
 a prefill after decode steps (a non-zero start position), dense and MoE.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -295,4 +297,37 @@ def test_speculative_verify(ctx, name, cfg, mode, seed):
     assert nxt == g[2]
     with pytest.raises(wpcg.WpcgError):
         m.set_position(n + 10)  # only backwards
+    m.close()
+
+
+def free_bytes():
+    hip = C.CDLL("libamdhip64.so")
+    free, total = C.c_size_t(), C.c_size_t()
+    assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def test_dense_batch_buffers_grow_with_the_prompt(ctx):
+    """A dense model's batch buffers hold 256 rows until a longer prompt comes;
+    then verification and a short prompt run on the larger ones. The wide MLP
+    makes the buffers what the free memory shows (per row 3 x 4 bytes an
+    intermediate value: 52 MB at 256 rows, 210 at 1024)."""
+    cfg = dict(DENSE, inter=17408, max_pos=640)
+    m = build(ctx, cfg, 41, wpcg.MODE_FAST)
+    toks = np.random.default_rng(41).integers(0, cfg["vocab"], 600).astype(np.uint32)
+    before = free_bytes()
+    short = m.prefill(toks[:12])[0]
+    assert 40 << 20 < before - free_bytes() < 100 << 20
+    m.reset()
+    got = m.prefill(toks[:600])[0]
+    assert 125 << 20 < before - free_bytes() < 180 << 20
+    m.reset()
+    assert np.array_equal(m.prefill(toks[:12])[0], short)
+    rows = m.verify(toks[12:20], want_logits=True)[1]
+    m.reset()
+    m.set_prefill(False)
+    exp = m.prefill(toks[:20])[0]
+    assert np.max(np.abs(rows[-1] - exp)) <= TOL * (exp.max() - exp.min())
+    exp = m.prefill(toks[20:600])[0]
+    assert np.max(np.abs(got - exp)) <= TOL * (exp.max() - exp.min())
     m.close()

@@ -26,10 +26,12 @@ struct Layer {
     std::vector<uint8_t> experts_set;                              // 3 bits per expert
 };
 
-// Batch buffers of the FAST prefill, made by the first prefill call: rows
-// are the chunk's tokens (at most cap of them).
+// Batch buffers of the FAST prefill, made by the first prefill call and again
+// by one that wants more rows (make_prefill): rows are the chunk's tokens (at
+// most cap of them).
 struct Prefill {
     uint32_t cap = 0;
+    std::vector<void*> allocs;  // everything below but vlogits and vids
     float *x = nullptr, *xn = nullptr, *q = nullptr, *k = nullptr, *v = nullptr, *attn = nullptr;
     float *g = nullptr, *u = nullptr;           // dense MLP [cap][inter]
     float *r = nullptr, *w = nullptr;           // router logits [cap][E], weights [cap][top_k]
@@ -157,6 +159,7 @@ void free_model(wpcg_model* m)
     if (m->embed) wpcg_linear_destroy(m->embed);
     if (m->lm_head) wpcg_linear_destroy(m->lm_head);
     for (void* p : m->allocs) (void)hipFree(p);
+    for (void* p : m->pf.allocs) (void)hipFree(p);
     if (m->pin_out) (void)hipHostFree(m->pin_out);
     if (m->pin_tok) (void)hipHostFree(m->pin_tok);
 }
@@ -461,11 +464,15 @@ int enqueue_step(wpcg_model* m, int kind, hipStream_t s)
 // Rows of tokens per prefill pass; longer prompts run pass after pass. The
 // expert grouping holds PF_GROUP_MAXT tokens; a dense pass reads every
 // weight once for four times as many (the 19456 x 2560 gate and up of 1000
-// tokens: 4 x 87 us in passes of 256, 208 in one).
+// tokens: 4 x 87 us in passes of 256, 208 in one). A packed X stays below the
+// GEMM's buffer offsets (2^30 bytes).
 constexpr uint32_t PF_CAP_DENSE = 1024;
 uint32_t pf_cap(const wpcg_model_config& c)
 {
-    return std::min(c.n_experts ? (uint32_t)PF_GROUP_MAXT : PF_CAP_DENSE, c.max_pos);
+    if (c.n_experts) return std::min((uint32_t)PF_GROUP_MAXT, c.max_pos);
+    const uint64_t k = std::max<uint64_t>({c.hidden, (uint64_t)c.n_heads * c.head_dim, c.inter});
+    const uint64_t fit = ((1ull << 30) - 1) / (std::max<uint64_t>(k / 128, 1) * 4096) / 4 * 32;
+    return (uint32_t)std::min<uint64_t>({PF_CAP_DENSE, std::max<uint64_t>(fit, WPCG_VERIFY_MAX), c.max_pos});
 }
 
 // Whether the batched path covers this model: FAST attention's head shapes,
@@ -482,13 +489,16 @@ bool prefill_ok(const wpcg_model* m)
            c.moe_inter % 128 == 0;
 }
 
-int make_prefill(wpcg_model* m)
+// The batch buffers for passes of rows rows in the place of m->pf's; m->pf is
+// left as it is on failure.
+int make_prefill_rows(wpcg_model* m, uint32_t rows)
 {
-    Prefill& P = m->pf;
-    if (P.cap) return WPCG_OK;
     const wpcg_model_config& c = m->cfg;
+    Prefill P;
+    P.vlogits = m->pf.vlogits;
+    P.vids = m->pf.vids;
     WPCG_HIP(hipDeviceGetAttribute(&P.cus, hipDeviceAttributeMultiprocessorCount, m->ctx->device));
-    const size_t cap = pf_cap(c), H = c.hidden, qd = (size_t)c.n_heads * c.head_dim,
+    const size_t cap = rows, H = c.hidden, qd = (size_t)c.n_heads * c.head_dim,
                  kvd = (size_t)c.n_kv_heads * c.head_dim;
     int rc = WPCG_OK;
     auto dev = [&](void** p, size_t bytes) {
@@ -498,7 +508,7 @@ int make_prefill(wpcg_model* m)
             rc = hip_fail(e, "prefill buffers");
             return;
         }
-        m->allocs.push_back(*p);
+        P.allocs.push_back(*p);
     };
     dev((void**)&P.x, cap * H * 4);
     dev((void**)&P.xn, cap * H * 4);
@@ -528,8 +538,28 @@ int make_prefill(wpcg_model* m)
         dev((void**)&P.g, cap * c.inter * 4);
         dev((void**)&P.u, cap * c.inter * 4);
     }
-    if (rc == WPCG_OK) P.cap = (uint32_t)cap;
-    return rc;
+    if (rc != WPCG_OK) {
+        for (void* p : P.allocs) (void)hipFree(p);
+        (void)hipGetLastError();
+        return rc;
+    }
+    P.cap = rows;
+    if (!m->pf.allocs.empty()) WPCG_HIP(hipStreamSynchronize(m->ctx->stream));
+    for (void* p : m->pf.allocs) (void)hipFree(p);
+    m->pf = std::move(P);
+    return WPCG_OK;
+}
+
+// Batch buffers for n tokens: a dense model's are made for PF_CAP_LEAST rows
+// until a longer prompt comes (Qwen3-4B shape: 43 MB, 170 MB for
+// PF_CAP_DENSE), which runs in passes of those where the memory for more is
+// not there.
+constexpr uint32_t PF_CAP_LEAST = 256;
+int make_prefill(wpcg_model* m, uint32_t n)
+{
+    const uint32_t most = pf_cap(m->cfg), least = std::min(most, PF_CAP_LEAST);
+    return grow_rows(m->pf.cap, n > least ? most : least, least,
+                     [&](uint32_t rows) { return make_prefill_rows(m, rows); });
 }
 
 // Tokens tokens[pos0 .. pos0+n-1] (already on the device) through every
@@ -611,7 +641,7 @@ int prefill_pass(wpcg_model* m, uint32_t pos0, uint32_t n, hipStream_t s)
 // the caller's n_prompt, so the argmax lands in tokens[] as a step's would).
 int prefill_run(wpcg_model* m, uint32_t pos0, uint32_t n, uint32_t n_prompt)
 {
-    if (int rc = make_prefill(m)) return rc;
+    if (int rc = make_prefill(m, n)) return rc;
     hipStream_t s = m->ctx->stream;
     const wpcg_model_config& c = m->cfg;
     uint32_t last = 0;
@@ -641,15 +671,17 @@ int prefill_run(wpcg_model* m, uint32_t pos0, uint32_t n, uint32_t n_prompt)
 // argmax; the position ends at pos0 + n with the last argmax as st.last.
 int verify_run(wpcg_model* m, uint32_t pos0, uint32_t n)
 {
-    if (int rc = make_prefill(m)) return rc;
+    if (int rc = make_prefill(m, n)) return rc;
     const wpcg_model_config& c = m->cfg;
     Prefill& P = m->pf;
     hipStream_t s = m->ctx->stream;
     if (!P.vlogits) {
+        if (!P.vids) {  // (the small one may be left from a call that could not have the other)
+            WPCG_HIP(hipMalloc(&P.vids, WPCG_VERIFY_MAX * 4));
+            m->allocs.push_back(P.vids);
+        }
         WPCG_HIP(hipMalloc(&P.vlogits, (size_t)WPCG_VERIFY_MAX * c.vocab * 4));
         m->allocs.push_back(P.vlogits);
-        WPCG_HIP(hipMalloc(&P.vids, WPCG_VERIFY_MAX * 4));
-        m->allocs.push_back(P.vids);
     }
     if (int rc = prefill_pass(m, pos0, n, s)) return rc;
     wpcg_linear* head = logits_head(m);

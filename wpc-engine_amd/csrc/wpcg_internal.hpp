@@ -430,7 +430,18 @@ hipError_t launch_pf_router(const float* X, const float* W, int T, int E, int K,
 // (token, slot) pairs sorted by expert for launch_gemm_grouped: pair_tok
 // [P], pair_pos [P], items [3 * (P / GEMM_GROUP_COLS + E)], nitems [1].
 constexpr int PF_MAX_PAIRS = 8192;
-constexpr int PF_GROUP_MAXT = 256;  // tokens per grouping (the prefill pass holds at most 256 rows)
+// Batch buffers of `have` rows against a call that wants `want`: make(rows)
+// (WPCG_OK or an error, then nothing changed) is asked for want rows; where
+// that fails, those there serve on, or least rows do if there are none.
+template <class Make>
+int grow_rows(uint32_t have, uint32_t want, uint32_t least, Make make)
+{
+    if (have >= want) return WPCG_OK;
+    const int rc = make(want);
+    if (rc == WPCG_OK || have > 0) return WPCG_OK;
+    return want > least ? make(least) : rc;
+}
+constexpr int PF_GROUP_MAXT = 256;  // tokens per grouping: a MoE prefill pass
 hipError_t launch_pf_group(const int32_t* ids, int P, int E, int top_k, int* pair_tok, int* pair_pos, int* items,
                            int* nitems, hipStream_t s);
 hipError_t launch_pf_combine(float* X, const float* D, const float* w, const int* pair_pos, int T, int top_k, int H,
