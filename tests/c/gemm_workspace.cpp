@@ -72,7 +72,7 @@ hipError_t launch_gemm(const DeviceMatrix&, const GemmWork&, const void*, int, i
     return hipSuccess;
 }
 hipError_t launch_gemm_wide(const DeviceMatrix&, void* xf, float* xsum, int tiles, const void*, int, uint32_t M,
-                            const float*, const float*, float*, hipStream_t)
+                            const float*, float*, float*, uint64_t, hipStream_t)
 {
     launched.push_back({xf, xsum, tiles, M});
     return hipSuccess;

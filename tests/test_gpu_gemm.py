@@ -237,9 +237,17 @@ def test_gemm_split_every_ksplit(ctx, M):
 # W, odd and even block counts on both sides of the K groups (1, 2, 4, 8), and
 # every workgroup shape (outputs from one tile to more than the chip).
 # 2^-17 and 3e-5 of the term sum as in the bounds above.
-@pytest.mark.parametrize("scheme,rows,cols,M", [
+MANY_ROWS = [
     (4, 1, 128, 65), (3, 33, 256, 95), (4, 16, 384, 96), (3, 300, 1152, 129), (4, 700, 1280, 100),
-    (3, 4864, 896, 300), (4, 9728, 640, 500), (3, 2560, 2560, 97), (4, 513, 4224, 1025), (4, 8192, 256, 2080)])
+    (3, 4864, 896, 300), (4, 9728, 640, 500), (3, 2560, 2560, 97), (4, 513, 4224, 1025), (4, 8192, 256, 2080)]
+# and with K in slices over workgroups: long rows of few outputs, an odd count
+# of blocks, a last slice shorter than the others
+K_SLICED = [
+    (4, 300, 128 * 77, 70), (3, 300, 128 * 77, 66), (4, 513, 12288, 100), (3, 16, 128 * 65, 65), (4, 2500, 9728, 65),
+    (3, 2500, 9728, 65)]
+
+
+@pytest.mark.parametrize("scheme,rows,cols,M", MANY_ROWS + K_SLICED)
 @pytest.mark.parametrize("dtype", [wpcg.DTYPE_BF16, wpcg.DTYPE_F32, wpcg.DTYPE_F32_SPLIT])
 def test_gemm_many_rows(ctx, scheme, rows, cols, M, dtype):
     print(f"[gpu] gemm v{scheme} {rows}x{cols} M={M} dtype={dtype}", flush=True)

@@ -23,20 +23,27 @@ void free_gemm(GemmWork& w)
 
 namespace {
 
+// Floats of the K-slices' partials (0: no kernel of this matrix has slices).
+uint64_t part_floats(const DeviceMatrix& m, const GemmWork& w)
+{
+    if (w.kg <= 1 && w.kg_small <= 1) return 0;
+    return std::max<uint64_t>((uint64_t)w.kg * GEMM_MAX_M, (uint64_t)w.kg_small * 16) * m.rows_pad;
+}
+
 int make_gemm(wpcg_linear* L, hipStream_t s)
 {
     const DeviceMatrix& m = L->m;
     GemmWork& w = L->gemm;
     w.kg = gemm_kslices(m.rows, m.nb, w.kg_req);
     w.kg_small = gemm_small_kslices(m.rows, m.nb, w.kg_req);
-    const uint64_t part = std::max<uint64_t>((uint64_t)w.kg * GEMM_MAX_M, (uint64_t)w.kg_small * 16) * m.rows_pad;
+    const uint64_t part = part_floats(m, w);
     // partial sums are addressed with 32-bit byte offsets
     if (part * 4 >= (1ull << 31))
         return fail(WPCG_E_SHAPE, "batched GEMM: too many rows for the split-K workspace");
     const uint64_t rgs = (uint64_t)std::max(gemm_row_groups(m.rows), gemm_small_row_groups(m.rows));
     hipError_t e = hipMalloc(&w.xf, m.nb * 4 * 4096);
     if (e == hipSuccess) e = hipMalloc(&w.xsum, m.nb * GEMM_MAX_M * sizeof(float));
-    if (e == hipSuccess && (w.kg > 1 || w.kg_small > 1)) e = hipMalloc(&w.part, part * sizeof(float));
+    if (e == hipSuccess && part) e = hipMalloc(&w.part, part * sizeof(float));
     if (e == hipSuccess) e = hipMalloc(&w.counters, std::max<uint64_t>(1, rgs) * sizeof(uint32_t));
     if (e == hipSuccess) e = hipMemsetAsync(w.counters, 0, std::max<uint64_t>(1, rgs) * sizeof(uint32_t), s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
@@ -62,7 +69,7 @@ bool wide(const wpcg_linear* L, int x_mode, uint32_t M)
 // While a graph is being captured, or where the memory is not there, the
 // largest one made, or the 64-column workspace, serves in smaller passes,
 // with the same results.
-int run_wide(wpcg_linear* L, const void* x, int x_mode, uint32_t M, const float* res, float* y, hipStream_t s)
+int run_wide(wpcg_linear* L, const void* x, int x_mode, uint32_t M, float* y, hipStream_t s)
 {
     const DeviceMatrix& m = L->m;
     GemmWork& w = L->gemm;
@@ -86,7 +93,7 @@ int run_wide(wpcg_linear* L, const void* x, int x_mode, uint32_t M, const float*
     const int tiles = i < 0 ? GEMM_MAX_M / 16 : gemm_wide_step(i);
     void* xf = i < 0 ? w.xf : w.wide[i];
     float* xsum = i < 0 ? w.xsum : reinterpret_cast<float*>(static_cast<uint8_t*>(xf) + m.nb * tiles * 4096);
-    WPCG_HIP(launch_gemm_wide(m, xf, xsum, tiles, x, x_mode, M, L->bias, res, y, s));
+    WPCG_HIP(launch_gemm_wide(m, xf, xsum, tiles, x, x_mode, M, L->bias, y, w.part, part_floats(m, w), s));
     return WPCG_OK;
 }
 
@@ -109,7 +116,7 @@ int run_gemm(wpcg_linear* L, const void* x, int x_dtype, uint32_t M, float* y, h
                                     "make it before capturing a graph");
         if (int rc = make_gemm(L, s)) return rc;
     }
-    if (wide(L, x_dtype, M)) return run_wide(L, x, x_dtype, M, nullptr, y, s);
+    if (wide(L, x_dtype, M)) return run_wide(L, x, x_dtype, M, y, s);
     const uint64_t es = x_dtype == WPCG_DTYPE_BF16 ? 2 : 4;
     const uint32_t step = x_dtype == WPCG_DTYPE_F32_SPLIT ? GEMM_MAX_M_SPLIT : GEMM_MAX_M;
     for (uint32_t c = 0; c < M; c += step) {
@@ -163,15 +170,12 @@ int wpcg_linear_gemm_noalloc(wpcg_linear* L, const void* x, int x_dtype, uint32_
     w.kg_small = gemm_small_kslices(m.rows, m.nb, w.kg_req);
     const uint64_t ncnt = std::max<uint64_t>(
         1, (uint64_t)std::max(gemm_row_groups(m.rows), gemm_small_row_groups(m.rows)));
-    const uint64_t part = (w.kg > 1 || w.kg_small > 1)
-                              ? std::max<uint64_t>((uint64_t)w.kg * GEMM_MAX_M, (uint64_t)w.kg_small * 16) *
-                                    m.rows_pad * sizeof(float)
-                              : 0;
+    const uint64_t part = part_floats(m, w) * sizeof(float);
     auto up = [](uint64_t b) { return (b + 255) / 256 * 256; };
-    const uint64_t o_xsum = up(ncnt * sizeof(uint32_t));
+    const uint64_t o_part = up(ncnt * sizeof(uint32_t));
+    const uint64_t o_xsum = o_part + up(part);
     const uint64_t o_xf = o_xsum + up(m.nb * GEMM_MAX_M * sizeof(float));
-    const uint64_t o_part = o_xf + up(m.nb * 4 * 4096);
-    const uint64_t need = o_part + up(part);
+    const uint64_t need = o_xf + up(m.nb * 4 * 4096);
     if (need > WPCG_NOALLOC_SCRATCH_BYTES)
         return fail(WPCG_E_UNSUPPORTED, "batched GEMM without allocation: this matrix needs " + std::to_string(need) +
                                             " bytes of workspace, the fixed array holds " +
@@ -183,10 +187,10 @@ int wpcg_linear_gemm_noalloc(wpcg_linear* L, const void* x, int x_dtype, uint32_
     w.xf = base + o_xf;
     w.part = part ? reinterpret_cast<float*>(base + o_part) : nullptr;
     if (wide(L, x_dtype, M)) {  // as many 16-column tiles as the array holds packed, a multiple of 4
-        const uint64_t room = WPCG_NOALLOC_SCRATCH_BYTES - up(ncnt * sizeof(uint32_t));
+        const uint64_t room = WPCG_NOALLOC_SCRATCH_BYTES - o_xsum;
         const int tiles = (int)std::min<uint64_t>(GEMM_WIDE_TILES, room / (m.nb * (4096 + 64)) / 4 * 4);
         w.xf = base + o_xsum + up(m.nb * tiles * 64);
-        WPCG_HIP(launch_gemm_wide(m, w.xf, w.xsum, tiles, x, x_dtype, M, L->bias, nullptr, y, s));
+        WPCG_HIP(launch_gemm_wide(m, w.xf, w.xsum, tiles, x, x_dtype, M, L->bias, y, w.part, part_floats(m, w), s));
         return WPCG_OK;
     }
     // the array keeps the last call's contents: the counters must start at 0

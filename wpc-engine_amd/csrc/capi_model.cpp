@@ -40,6 +40,7 @@ struct Prefill {
     float *ge = nullptr, *ue = nullptr, *de = nullptr;  // per sorted pair: [P][moe_inter] x2, [P][hidden]
     void* xf = nullptr;       // packed X of the batched GEMMs (launch_gemm_pack_rows)
     float* xsum = nullptr;
+    float* part = nullptr;    // o_proj's and the dense down's K-slices, PF_PART floats
     int cus = 0;              // the device's CUs: the expert-grouped GEMMs' workgroups
     void* dg = nullptr;       // the expert-grouped GEMMs' X digits (launch_pf_digits)
     float* dxs = nullptr;
@@ -489,6 +490,11 @@ bool prefill_ok(const wpcg_model* m)
            c.moe_inter % 128 == 0;
 }
 
+// Floats for the K-slices of the projections into the residual: 256
+// workgroups of the shape that small launches take (64 x 32 outputs) and twice
+// as much again.
+constexpr uint64_t PF_PART = 3 * 256 * 64 * 32;
+
 // The batch buffers for passes of rows rows in the place of m->pf's; m->pf is
 // left as it is on failure.
 int make_prefill_rows(wpcg_model* m, uint32_t rows)
@@ -519,6 +525,7 @@ int make_prefill_rows(wpcg_model* m, uint32_t rows)
     const size_t kmax = std::max<size_t>({H, qd, c.n_experts ? 0 : (size_t)c.inter});
     dev((void**)&P.xf, kmax / 128 * gemm_rows_tiles((int)cap) * 4096);
     dev((void**)&P.xsum, kmax / 128 * gemm_rows_tiles((int)cap) * 16 * 4);
+    dev((void**)&P.part, PF_PART * 4);
     if (c.n_experts) {
         const size_t pairs = cap * c.top_k, E = c.n_experts, I = c.moe_inter;
         dev((void**)&P.r, cap * E * 4);
@@ -598,7 +605,7 @@ int prefill_pass(wpcg_model* m, uint32_t pos0, uint32_t n, hipStream_t s)
             const DeviceMatrix* ms[1] = {&l->m};
             const float* bs[1] = {l->bias};
             float* ys[1] = {P.x};
-            return launch_gemm_packed_rows(ms, bs, ys, 1, P.xf, P.xsum, (int)n, P.x, s);
+            return launch_gemm_packed_rows(ms, bs, ys, 1, P.xf, P.xsum, (int)n, P.x, s, nullptr, P.part, PF_PART);
         };
         WPCG_HIP(residual(L.o));
         if (!c.n_experts) {

@@ -464,7 +464,7 @@ __global__ __launch_bounds__(GM_WG) void k_gemm(const GemmArgs P)
         }
 }
 
-// The split-K sum of k_gemm: Y[m][row] = sum over the kg slices of
+// The split-K sum of k_gemm and k_gemm_wide: Y[m][row] = sum over the kg slices of
 // part[k][m][row] in slice order, then the bias and the residual. One thread
 // per four rows of one column; reads and writes run along the rows.
 __global__ __launch_bounds__(256) void k_gemm_reduce(const float* __restrict__ part, int kg, int Mp, int rows_pad,
@@ -1240,9 +1240,17 @@ hipError_t launch_gemm(const DeviceMatrix& m, const GemmWork& w, const void* x, 
     if (split) e = m.scheme == 4 ? launch_nt<4, true>(ntiles, grid, s, a) : launch_nt<3, true>(ntiles, grid, s, a);
     else e = m.scheme == 4 ? launch_nt<4, false>(ntiles, grid, s, a) : launch_nt<3, false>(ntiles, grid, s, a);
     if (e != hipSuccess || w.kg == 1) return e;
-    const int outs = M * (int)(m.rows_pad / 4);
-    hipLaunchKernelGGL(k_gemm_reduce, dim3((unsigned)((outs + 255) / 256)), dim3(256), 0, s, w.part, w.kg,
-                       ntiles * 16, (int)m.rows_pad, (int)m.rows, M, bias, res, y);
+    return launch_gemm_reduce(w.part, w.kg, ntiles * 16, (int)m.rows_pad, (int)m.rows, M, bias, res, y, s);
+}
+
+hipError_t launch_gemm_reduce(const float* part, int kg, int Mp, int rows_pad, int rows, int M, const float* bias,
+                              const float* res, float* y, hipStream_t s)
+{
+    const int64_t outs = (int64_t)M * (rows_pad / 4);
+    if (M < 1 || M > Mp || kg < 1 || rows_pad % 4 || outs > INT32_MAX - 256) return hipErrorInvalidValue;
+    (void)hipGetLastError();
+    hipLaunchKernelGGL(k_gemm_reduce, dim3((unsigned)((outs + 255) / 256)), dim3(256), 0, s, part, kg, Mp, rows_pad,
+                       rows, M, bias, res, y);
     return hipGetLastError();
 }
 

@@ -30,6 +30,7 @@
 
 #include <algorithm>
 
+#include "wide_shape.h"
 #include "wpcg_internal.hpp"
 #include "xpack.h"
 
@@ -55,7 +56,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void* base, int
 }
 constexpr int PAST = 1 << 30;  // added to a buffer offset: past every range, reads zero (ranges are shorter)
 
-// One matrix of a launch: its tiles are t0 .. t0 + rgs * cgs - 1.
+// One matrix of a launch: its tiles (times kg slices) start at t0.
 struct WideMat {
     const uint8_t* codes;
     const uint8_t* hp;
@@ -73,7 +74,8 @@ struct WideArgs {
     const u32x4* xf;    // packed X, [nb][xt][4][64] fragments
     const float* xsum;  // [nb][xt*16]
     const float* res;   // [M][rows] added to Y (may be y itself) or null (one matrix only)
-    int nmat, nb, M, xt, cgs, total;
+    float* part;        // kg > 1: [kg][M][rows_pad] sums of the K-slices (one matrix only)
+    int nmat, nb, M, xt, cgs, total, kg, nbk;  // nbk: blocks of a slice
     // rope: the rotation tables and positions of the rows of X
     const float* cos_t;  // [max_pos][64]
     const float* sin_t;
@@ -118,13 +120,22 @@ __device__ __forceinline__ bf16x8 codes_bf16(uint32_t a, uint32_t b)
 // (two buffers, one barrier a round), fetched into registers a round ahead,
 // the codes straight into registers two rounds ahead.
 //
+// KS also splits K over kg workgroups, where even so there are too few (2560
+// weight rows and 24 rows of X are 40 workgroups of the smallest shape): each
+// takes a run of blocks and leaves its sums in part, which the next launch
+// (launch_gemm_reduce) adds in slice order: o_proj and down of a 24-token
+// Qwen3-4B-shaped prompt 51.6 us together without slices, 24.3 and 8.8 for the
+// reduces with them; 512 x 12288 at 33 rows SPLIT 39.6 -> 23.7 us a call. (A
+// form of its own: with the slice in the other launches too, the small v3
+// ones were 1 us slower.)
+//
 // ROPE (the prefill's q, k and v; WR % 4 == 0): four row tiles are one
 // 128-wide head. The sums go to LDS as [token][d], and 16 threads take a
 // token of a head: the head RMSNorm (FAST: squares by fused multiply-adds,
 // then exchanges), (x * scale) * w, the rotation at the token's position
 // (d < 64 and d + 64 are a pair: y c - y' s and y' c + y s), q into Y, k
 // and v (v as computed) into the cache rows, all as 16-byte pieces.
-template <int SCHEME, bool SPLIT, int CT, int WR, int WC, int KW, bool ROPE>
+template <int SCHEME, bool SPLIT, int CT, int WR, int WC, int KW, bool ROPE, bool KS>
 __global__ __launch_bounds__(WR * WC * KW * 64, WR * WC * KW == 16 ? 4 : 2) void k_gemm_wide(const WideArgs P0)
 {
     constexpr int WG = WR * WC * KW * 64;
@@ -150,27 +161,31 @@ __global__ __launch_bounds__(WR * WC * KW * 64, WR * WC * KW == 16 ? 4 : 2) void
     for (int i = 1; i < P0.nmat; i++) e = t >= P0.mat[i].t0 ? i : e;
     const WideMat P = P0.mat[e];
     const int tl = t - P.t0;
-    const int rg = __builtin_amdgcn_readfirstlane(tl / P0.cgs), cg = tl - rg * P0.cgs;  // the division runs on lanes
-    const int nb = P0.nb, XT = P0.xt;
+    const int rk = __builtin_amdgcn_readfirstlane(tl / P0.cgs), cg = tl - rk * P0.cgs;  // the division runs on lanes
+    const int rg = KS ? __builtin_amdgcn_readfirstlane(rk / P0.kg) : rk, ks = KS ? rk - rg * P0.kg : 0;
+    const int nbt = P0.nb, XT = P0.xt;
+    const int b0 = KS ? ks * P0.nbk : 0, nb = KS ? min(P0.nbk, nbt - b0) : nbt;  // the slice (none is empty)
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int kw = wave / (WR * WC), wrc = wave % (WR * WC), wr = wrc / WC, wc = wrc % WC;
     const int half = lane >> 5, jj = lane & 31, j = jj & 15;
     const int ntiles = P.rows_pad / TILE_ROWS;
     const int T0 = (rg * WR + wr) * 2;  // the wave's first 16-row tile
     const int live = __builtin_amdgcn_readfirstlane(max(0, min(2, ntiles - T0)));
-    const size_t rec0 = (size_t)min(T0, ntiles - 1) * nb;
-    const auto crs = buf_rsrc(P.codes + rec0 * CODE_REC, live * nb * (int)CODE_REC);
-    const auto hrs = buf_rsrc((SCHEME == 3 ? P.hp : P.codes) + rec0 * HP_REC, SCHEME == 3 ? live * nb * (int)HP_REC : 0);
-    const auto prs = buf_rsrc(P.params + rec0 * TILE_ROWS, live * nb * TILE_ROWS * 4);
-    const auto xrs = buf_rsrc(P0.xf, nb * XT * 4096);
-    const auto srs = buf_rsrc(P0.xsum, nb * XT * 64);
+    // (every range starts at the slice's first block and ends with the second tile's slice)
+    const size_t rec0 = (size_t)min(T0, ntiles - 1) * nbt + b0;
+    const int recs = !KS ? live * nb : live ? (live - 1) * nbt + nb : 0;
+    const auto crs = buf_rsrc(P.codes + rec0 * CODE_REC, recs * (int)CODE_REC);
+    const auto hrs = buf_rsrc((SCHEME == 3 ? P.hp : P.codes) + rec0 * HP_REC, SCHEME == 3 ? recs * (int)HP_REC : 0);
+    const auto prs = buf_rsrc(P.params + rec0 * TILE_ROWS, recs * TILE_ROWS * 4);
+    const auto xrs = buf_rsrc(P0.xf + (size_t)b0 * XT * 256, nb * XT * 4096);
+    const auto srs = buf_rsrc(P0.xsum + (size_t)b0 * XT * 16, nb * XT * 64);
 
     // the wave's codes of one block: word ga is lane group g = 2 ga + half of
     // 16-row tile jj / 16
     u32x4 cw[2][2];
     u32x2 hw[2][2];
     uint32_t pw[2];
-    const int crec = (jj >> 4) * nb;  // record of block 0
+    const int crec = (jj >> 4) * nbt;  // record of block 0
     auto load_word = [&](int u, int ga, int b) {
         const int past = b < nb ? 0 : PAST;
         cw[u][ga] = __builtin_amdgcn_raw_buffer_load_b128(
@@ -376,6 +391,17 @@ __global__ __launch_bounds__(WR * WC * KW * 64, WR * WC * KW == 16 ? 4 : 2) void
         }
         return;
     }
+    if constexpr (KS) {
+        if (row >= P.rows_pad) return;
+#pragma unroll
+        for (int ct = 0; ct < CT; ct++)
+#pragma unroll
+            for (int q = 0; q < 16; q++) {
+                const int m = ((cg * WC + wc) * CT + ct) * 32 + 8 * (q >> 2) + 4 * half + (q & 3);
+                if (m < P0.M) P0.part[((size_t)ks * P0.M + m) * P.rows_pad + row] = acc[ct][q];
+            }
+        return;
+    }
     if (row >= P.rows) return;
     const float bias = P.bias ? P.bias[row] : 0.0f;
 #pragma unroll
@@ -393,7 +419,7 @@ __global__ __launch_bounds__(WR * WC * KW * 64, WR * WC * KW == 16 ? 4 : 2) void
 }
 
 
-template <int SCHEME, bool SPLIT, int CT, int WR, int WC, int KW, bool ROPE = false>
+template <int SCHEME, bool SPLIT, int CT, int WR, int WC, int KW, bool ROPE = false, bool KS = false>
 hipError_t launch_cfg(WideArgs a, hipStream_t s)
 {
     a.cgs = ((a.M + 31) / 32 + CT * WC - 1) / (CT * WC);
@@ -402,53 +428,35 @@ hipError_t launch_cfg(WideArgs a, hipStream_t s)
         WideMat& m = a.mat[e];
         m.rgs = ((m.rows_pad + 31) / 32 + WR - 1) / WR;
         m.t0 = a.total;
-        a.total += m.rgs * a.cgs;
+        a.total += m.rgs * a.cgs * a.kg;
     }
-    hipLaunchKernelGGL((k_gemm_wide<SCHEME, SPLIT, CT, WR, WC, KW, ROPE>), dim3((unsigned)((a.total + 7) / 8 * 8)),
+    hipLaunchKernelGGL((k_gemm_wide<SCHEME, SPLIT, CT, WR, WC, KW, ROPE, KS>), dim3((unsigned)((a.total + 7) / 8 * 8)),
                        dim3(WR * WC * KW * 64), 0, s, a);
     return hipGetLastError();
 }
 
-// A tile shape: 32-row and 32-column tiles of a workgroup, and what one
-// K-block of a round of 256 workgroups takes in hundredths of a microsecond
-// (v4, v3), measured over 512..15360 rows, K 768..15360 and 40..1024 rows of
-// X; the shape with the fewest rounds x time wins. Large outputs fill the
-// chip with the widest tile (15360 x 3840, 1024 rows: 256 x 128 144 us,
-// 128 x 64 164, 64 x 32 357), small ones need the narrow, K-split ones
-// (3840 x 15360, 128 rows: 64 x 32 37 us, 128 x 64 97, 256 x 128 197).
-struct Shape {
-    int rows32, cols32;
-    int cost[2];
-    bool shared;  // workgroups of 8 waves share a CU: the chip fills by fractions of a round
-};
-
-int pick(const Shape* sh, int n, const WideArgs& a, int cols32, int scheme)
-{
-    int best = 0;
-    int64_t best_t = INT64_MAX;
-    for (int i = 0; i < n; i++) {
-        int64_t wgs = 0;
-        for (int e = 0; e < a.nmat; e++) wgs += ((a.mat[e].rows_pad + 31) / 32 + sh[i].rows32 - 1) / sh[i].rows32;
-        wgs *= (cols32 + sh[i].cols32 - 1) / sh[i].cols32;
-        const int64_t c = sh[i].cost[scheme == 3];
-        const int64_t t = sh[i].shared ? std::max(c * 4 / 3 * 256, c * (wgs + 128)) : (wgs + 255) / 256 * 256 * c;
-        if (t < best_t) {
-            best_t = t;
-            best = i;
-        }
-    }
-    return best;
-}
-
-// M: the rows of X that pick the shape (the whole batch of a pass)
+// M: the rows of X that pick the shape (the whole batch of a pass); part
+// holds part_floats, for K-slices
 template <int SCHEME, bool SPLIT>
-hipError_t launch_any(const WideArgs& a, uint32_t M, bool rope, hipStream_t s)
+hipError_t launch_any(WideArgs& a, uint32_t M, bool rope, float* part, uint64_t part_floats, hipStream_t s)
 {
-    const int cols32 = (int)((M + 31) / 32);
+    int tiles32[WIDE_MATS] = {};
+    for (int e = 0; e < a.nmat; e++) tiles32[e] = (a.mat[e].rows_pad + 31) / 32;
+    const WidePick p = pick_wide(SPLIT, rope, SCHEME, tiles32, a.nmat, (int)((M + 31) / 32), a.nb,
+                                 (uint64_t)M * a.mat[0].rows_pad, part ? part_floats : 0);
+    a.kg = p.kg;
+    a.nbk = (a.nb + p.kg - 1) / p.kg;
+    a.part = part;
+    if (p.kg > 1) {  // (pick_wide slices these two only)
+        if constexpr (!SPLIT)
+            return p.shape == 3 ? launch_cfg<SCHEME, SPLIT, 1, 4, 1, 4, false, true>(a, s)
+                                : launch_cfg<SCHEME, SPLIT, 1, 2, 1, 8, false, true>(a, s);
+        else
+            return p.shape == 3 ? launch_cfg<SCHEME, SPLIT, 1, 4, 1, 4, false, true>(a, s)
+                                : launch_cfg<SCHEME, SPLIT, 1, 2, 1, 4, false, true>(a, s);
+    }
     if constexpr (!SPLIT) {
-        static constexpr Shape sh[] = {{8, 4, {200, 220}, false}, {4, 2, {62, 69}, true}, {4, 2, {70, 80}, false},
-                                       {4, 1, {39, 60}, false}, {2, 1, {33, 57}, false}};
-        switch (pick(sh, 5, a, cols32, SCHEME)) {
+        switch (p.shape) {
         case 0: return launch_cfg<SCHEME, SPLIT, 2, 8, 2, 1>(a, s);
         case 1: return launch_cfg<SCHEME, SPLIT, 1, 4, 2, 1>(a, s);
         case 2: return launch_cfg<SCHEME, SPLIT, 1, 4, 2, 2>(a, s);
@@ -456,12 +464,8 @@ hipError_t launch_any(const WideArgs& a, uint32_t M, bool rope, hipStream_t s)
         default: return launch_cfg<SCHEME, SPLIT, 1, 2, 1, 8>(a, s);
         }
     } else {
-        // (the last one has no whole heads: not for rope)
-        static constexpr Shape sh[] = {{16, 1, {160, 165}, false}, {4, 2, {110, 118}, true}, {4, 2, {100, 110}, false},
-                                       {4, 1, {65, 80}, false}, {8, 1, {88, 105}, false}, {2, 1, {60, 70}, false}};
-        const int c = pick(sh, rope ? 5 : 6, a, cols32, SCHEME);
         if (rope) {
-            switch (c) {
+            switch (p.shape) {
             case 0: return launch_cfg<SCHEME, SPLIT, 1, 16, 1, 1, true>(a, s);
             case 1: return launch_cfg<SCHEME, SPLIT, 1, 4, 2, 1, true>(a, s);
             case 2: return launch_cfg<SCHEME, SPLIT, 1, 4, 2, 2, true>(a, s);
@@ -469,7 +473,7 @@ hipError_t launch_any(const WideArgs& a, uint32_t M, bool rope, hipStream_t s)
             default: return launch_cfg<SCHEME, SPLIT, 1, 8, 1, 2, true>(a, s);
             }
         }
-        switch (c) {
+        switch (p.shape) {
         case 0: return launch_cfg<SCHEME, SPLIT, 1, 16, 1, 1>(a, s);
         case 1: return launch_cfg<SCHEME, SPLIT, 1, 4, 2, 1>(a, s);
         case 2: return launch_cfg<SCHEME, SPLIT, 1, 4, 2, 2>(a, s);
@@ -478,6 +482,14 @@ hipError_t launch_any(const WideArgs& a, uint32_t M, bool rope, hipStream_t s)
         default: return launch_cfg<SCHEME, SPLIT, 1, 2, 1, 4>(a, s);
         }
     }
+}
+
+// The slices' sums, the bias and the residual into Y, where there are slices
+hipError_t finish(const WideArgs& a, hipStream_t s)
+{
+    const WideMat& m = a.mat[0];
+    if (a.kg == 1) return hipSuccess;
+    return launch_gemm_reduce(a.part, a.kg, a.M, m.rows_pad, m.rows, a.M, m.bias, a.res, m.y, s);
 }
 
 WideMat wide_mat(const DeviceMatrix& m, const float* bias, float* y)
@@ -496,7 +508,7 @@ WideMat wide_mat(const DeviceMatrix& m, const float* bias, float* y)
 }  // namespace
 
 hipError_t launch_gemm_wide(const DeviceMatrix& m, void* xf, float* xsum, int tiles, const void* x, int x_mode,
-                            uint32_t M, const float* bias, const float* res, float* y, hipStream_t s)
+                            uint32_t M, const float* bias, float* y, float* part, uint64_t part_floats, hipStream_t s)
 {
     const bool split = x_mode == GX_SPLIT;
     // (the shape is picked from the whole batch, so that the order of an
@@ -515,12 +527,14 @@ hipError_t launch_gemm_wide(const DeviceMatrix& m, void* xf, float* xsum, int ti
         a.nmat = 1;
         a.xf = static_cast<const u32x4*>(xf);
         a.xsum = xsum;
-        a.res = res ? res + (uint64_t)c * m.rows : nullptr;
         a.nb = (int)m.nb;
         a.M = mc;
         a.xt = xt;
-        if (split) e = m.scheme == 4 ? launch_any<4, true>(a, M, false, s) : launch_any<3, true>(a, M, false, s);
-        else e = m.scheme == 4 ? launch_any<4, false>(a, M, false, s) : launch_any<3, false>(a, M, false, s);
+        if (split) e = m.scheme == 4 ? launch_any<4, true>(a, M, false, part, part_floats, s)
+                                     : launch_any<3, true>(a, M, false, part, part_floats, s);
+        else e = m.scheme == 4 ? launch_any<4, false>(a, M, false, part, part_floats, s)
+                               : launch_any<3, false>(a, M, false, part, part_floats, s);
+        if (e == hipSuccess) e = finish(a, s);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
@@ -528,7 +542,7 @@ hipError_t launch_gemm_wide(const DeviceMatrix& m, void* xf, float* xsum, int ti
 
 hipError_t launch_gemm_packed_rows(const DeviceMatrix* const* ms, const float* const* biases, float* const* ys,
                                    int count, const void* xf, const float* xsum, int M, const float* res,
-                                   hipStream_t s, const GemmRope* rope)
+                                   hipStream_t s, const GemmRope* rope, float* part, uint64_t part_floats)
 {
     if (M < 1 || count < 1 || count > WIDE_MATS || (res && count > 1)) return hipErrorInvalidValue;
     if (ms[0]->nb * (uint64_t)gemm_rows_tiles(M) * 4096 >= (uint64_t)PAST) return hipErrorInvalidValue;
@@ -563,8 +577,9 @@ hipError_t launch_gemm_packed_rows(const DeviceMatrix* const* ms, const float* c
     a.nb = (int)ms[0]->nb;
     a.M = M;
     a.xt = gemm_rows_tiles(M);
-    return ms[0]->scheme == 4 ? launch_any<4, true>(a, (uint32_t)M, rope != nullptr, s)
-                              : launch_any<3, true>(a, (uint32_t)M, rope != nullptr, s);
+    const hipError_t e = ms[0]->scheme == 4 ? launch_any<4, true>(a, (uint32_t)M, rope != nullptr, part, part_floats, s)
+                                            : launch_any<3, true>(a, (uint32_t)M, rope != nullptr, part, part_floats, s);
+    return e == hipSuccess ? finish(a, s) : e;
 }
 
 }  // namespace wpcg

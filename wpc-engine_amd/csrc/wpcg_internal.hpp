@@ -238,8 +238,13 @@ hipError_t launch_gemm(const DeviceMatrix& m, const GemmWork& w, const void* x, 
 // does not depend on the passes it is split into.
 // GEMM_WIDE_TILES hold 2048 rows of X a pass, 1024 in the SPLIT mode.
 inline int gemm_wide_cols(int x_mode, int tiles) { return x_mode == GX_SPLIT ? tiles / 4 * 32 : tiles / 2 * 32; }
+// part (part_floats of them, may be null) holds the sums of K-slices.
 hipError_t launch_gemm_wide(const DeviceMatrix& m, void* xf, float* xsum, int tiles, const void* x, int x_mode,
-                            uint32_t M, const float* bias, const float* res, float* y, hipStream_t s);
+                            uint32_t M, const float* bias, float* y, float* part, uint64_t part_floats, hipStream_t s);
+// The K-slices' sums part [kg][Mp][rows_pad] in slice order, plus bias and
+// res, into y, rows of X m < M.
+hipError_t launch_gemm_reduce(const float* part, int kg, int Mp, int rows_pad, int rows, int M, const float* bias,
+                              const float* res, float* y, hipStream_t s);
 hipError_t launch_gemm_pack(const void* x, int x_mode, int M, int K, int xt, int nt, void* xf, float* xsum,
                             hipStream_t s);
 // Expert-grouped GEMM, one launch for every expert of a stack (or of two
@@ -270,7 +275,7 @@ hipError_t launch_gemm_pack_rows(const float* x, int M, int K, void* xf, float* 
 // of X are the tokens at positions pos0 ..): GEMM_ROPE_Q the head RMSNorm
 // (weights nw[e]) and the rotation (cos_t / sin_t [max_pos][64]) into Y,
 // GEMM_ROPE_K the same into cache[e] ([head][max_pos][128]), GEMM_ROPE_V the
-// rows as computed into cache[e].
+// rows as computed into cache[e]. part: as in launch_gemm_wide (one matrix).
 constexpr int GEMM_ROPE_Q = 1, GEMM_ROPE_K = 2, GEMM_ROPE_V = 3;
 struct GemmRope {
     int mode[3];
@@ -283,7 +288,8 @@ struct GemmRope {
 };
 hipError_t launch_gemm_packed_rows(const DeviceMatrix* const* ms, const float* const* biases, float* const* ys,
                                    int count, const void* xf, const float* xsum, int M, const float* res,
-                                   hipStream_t s, const GemmRope* rope = nullptr);
+                                   hipStream_t s, const GemmRope* rope = nullptr, float* part = nullptr,
+                                   uint64_t part_floats = 0);
 // The grouped GEMM's X: rows x rows of K fp32 (xu non-null: silu(x) * xu,
 // the FAST steps' arithmetic, xu of x's shape) to int8 digits, dg
 // rows * K * 4 bytes, and per 128-value block {s_b 2^-7, sum}, dxs
