@@ -49,7 +49,7 @@ def test_k_slices_where_half_the_chip_idles(pick):
             assert pick(split, 0, scheme, m, cols, 0, [rows])[1] == 1
             if k > 1:
                 seen.add((split, scheme, shape))
-    assert seen == {(p, s, h) for s in (3, 4) for p, h in ((0, 3), (0, 4), (1, 3), (1, 5))}
+    assert seen == {(p, s, h) for s in (3, 4) for p, h in ((0, 3), (0, 4), (1, 1), (1, 3))}
     # q, k and v together, or gate and up, have no slices
     assert pick(1, 1, 4, 24, 2560, 1 << 22, [4096, 1024, 1024])[1] == 1
     assert pick(1, 0, 4, 24, 12288, 1 << 22, [512, 512])[1] == 1

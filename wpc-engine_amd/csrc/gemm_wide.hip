@@ -452,7 +452,7 @@ hipError_t launch_any(WideArgs& a, uint32_t M, bool rope, float* part, uint64_t 
             return p.shape == 3 ? launch_cfg<SCHEME, SPLIT, 1, 4, 1, 4, false, true>(a, s)
                                 : launch_cfg<SCHEME, SPLIT, 1, 2, 1, 8, false, true>(a, s);
         else
-            return p.shape == 3 ? launch_cfg<SCHEME, SPLIT, 1, 4, 1, 4, false, true>(a, s)
+            return p.shape == 1 ? launch_cfg<SCHEME, SPLIT, 1, 4, 1, 4, false, true>(a, s)
                                 : launch_cfg<SCHEME, SPLIT, 1, 2, 1, 4, false, true>(a, s);
     }
     if constexpr (!SPLIT) {
@@ -467,19 +467,16 @@ hipError_t launch_any(WideArgs& a, uint32_t M, bool rope, float* part, uint64_t 
         if (rope) {
             switch (p.shape) {
             case 0: return launch_cfg<SCHEME, SPLIT, 1, 16, 1, 1, true>(a, s);
-            case 1: return launch_cfg<SCHEME, SPLIT, 1, 4, 2, 1, true>(a, s);
-            case 2: return launch_cfg<SCHEME, SPLIT, 1, 4, 2, 2, true>(a, s);
-            case 3: return launch_cfg<SCHEME, SPLIT, 1, 4, 1, 4, true>(a, s);
+            case 1: return launch_cfg<SCHEME, SPLIT, 1, 4, 1, 4, true>(a, s);
             default: return launch_cfg<SCHEME, SPLIT, 1, 8, 1, 2, true>(a, s);
             }
         }
         switch (p.shape) {
         case 0: return launch_cfg<SCHEME, SPLIT, 1, 16, 1, 1>(a, s);
-        case 1: return launch_cfg<SCHEME, SPLIT, 1, 4, 2, 1>(a, s);
-        case 2: return launch_cfg<SCHEME, SPLIT, 1, 4, 2, 2>(a, s);
-        case 3: return launch_cfg<SCHEME, SPLIT, 1, 4, 1, 4>(a, s);
-        case 4: return launch_cfg<SCHEME, SPLIT, 1, 8, 1, 2>(a, s);
-        default: return launch_cfg<SCHEME, SPLIT, 1, 2, 1, 4>(a, s);
+        case 1: return launch_cfg<SCHEME, SPLIT, 1, 4, 1, 4>(a, s);
+        case 2: return launch_cfg<SCHEME, SPLIT, 1, 8, 1, 2>(a, s);
+        case 3: return launch_cfg<SCHEME, SPLIT, 1, 2, 1, 4>(a, s);
+        default: return launch_cfg<SCHEME, SPLIT, 1, 4, 2, 2>(a, s);
         }
     }
 }

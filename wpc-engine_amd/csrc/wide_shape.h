@@ -24,10 +24,15 @@ struct WideShape {
 constexpr WideShape WIDE_BF16[] = {{8, 4, {200, 220}, false, false}, {4, 2, {62, 69}, true, false},
                                    {4, 2, {70, 80}, false, false},   {4, 1, {39, 60}, false, true},
                                    {2, 1, {33, 57}, false, true}};
-// (the last one has no whole heads: not for the q/k/v epilogue)
-constexpr WideShape WIDE_SPLIT[] = {{16, 1, {160, 165}, false, false}, {4, 2, {110, 118}, true, false},
-                                    {4, 2, {100, 110}, false, false},  {4, 1, {65, 80}, false, true},
-                                    {8, 1, {88, 105}, false, false},   {2, 1, {60, 70}, false, true}};
+// (128 x 64 in 8 waves is not among these: it holds 132-137 registers, so no two
+// of them share a CU, and where it was picked it took 5-18 % longer than what is
+// picked without it. The last two have no form for the q/k/v epilogue: no whole
+// heads, and no launch that would pick it.)
+constexpr WideShape WIDE_SPLIT[] = {{16, 1, {160, 165}, false, false},
+                                    {4, 1, {65, 80}, false, true},
+                                    {8, 1, {88, 105}, false, false},
+                                    {2, 1, {60, 70}, false, true},
+                                    {4, 2, {100, 110}, false, false}};
 
 // K-slices over workgroups, for launches that leave half of the chip idle
 // even in 64 x 32 tiles (SPLIT 3840 x 15360 v3, 96 rows, 180 such tiles: 49.4
@@ -47,11 +52,12 @@ struct WidePick {
 // tiles32: 32-row tiles of each of the nmat matrices; cols32: 32-row tiles of
 // X; nb: K-blocks; outs: outputs (rows of X times padded weight rows), whose
 // partials must fit part_floats (0: no slices).
+// rope (SPLIT only): with the q/k/v epilogue.
 inline WidePick pick_wide(bool split, bool rope, int scheme, const int* tiles32, int nmat, int cols32, int nb,
                           uint64_t outs, uint64_t part_floats)
 {
     const WideShape* sh = split ? WIDE_SPLIT : WIDE_BF16;
-    const int n = split ? (rope ? 5 : 6) : 5;
+    const int n = rope ? 3 : 5;
     int64_t small = 0;  // 64 x 32 tiles
     for (int e = 0; e < nmat; e++) small += (int64_t)((tiles32[e] + 1) / 2) * cols32;
     const int most = rope || nmat > 1 || small > 128
