@@ -51,8 +51,9 @@ ODD_OPROJ = dict(n_layers=2, hidden=256, n_heads=6, n_kv_heads=2, head_dim=64, i
 # The down projection's 97 blocks are four K-slices, which join inside its
 # launch: the residual's deferred o_proj slice has to be added there
 FOUR_SLICE_DOWN = dict(DENSE, inter=128 * 97)
-# Long contexts: past 16 x 32 = 512 positions each FAST attention chunk holds
-# a second block of 32 positions, past 1024 a third. LONG: head_dim 64 with
+# Long contexts: past 16 x 32 = 512 positions each of FAST attention's 16
+# chunks holds a second block of 32 positions; from 768 on there are 64 chunks
+# of one block (two past 2048: see the test of those). LONG: head_dim 64 with
 # 2 query heads per key head (the 512-thread attention); LONG_REP8: head_dim
 # 128 with 8 query heads per key head (the 256-thread attention, as in the
 # Qwen3-30B-A3B shape).
@@ -147,11 +148,11 @@ def test_exact_decode_is_bit_identical(ctx, name, cfg, n_prompt, n_new, seed):
 def test_fast_decode_tracks_the_reference(ctx, name, cfg, n_steps, seed):
     """FAST mode step by step on the oracle's greedy tokens: every step's
     logits within FAST_TOL of the logit range of the oracle's, and the same
-    argmax. The FAST attention splits the positions into blocks of 32, chunk
-    c holding blocks c, c + 16, ...; the steps cross many block boundaries
-    (and, in the long cases, the second and third rounds of blocks), so the
-    chunk merge, empty chunks and the key/value appends of every chunk are
-    exercised."""
+    argmax. The FAST attention deals the positions to its chunks in turn, and
+    a chunk takes them 32 at a time; the steps fill the chunks one after
+    another (and, in the long cases, cross into second blocks and into 64
+    chunks), so the chunk merge, empty chunks and the key/value appends of every
+    chunk are exercised."""
     print(f"[gpu] fast decode {name}: building", flush=True)
     m, ref = build(ctx, cfg, seed)
     m.set_mode(wpcg.MODE_FAST)
@@ -195,6 +196,29 @@ def test_fast_steps_across_the_long_context_line(ctx, name, cfg):
     m.set_position(766)
     got += [m.forward_token(int(t))[0] for t in toks[766:770]]
     for g, r in zip(got, exp[764:] + exp[766:770]):
+        assert float(np.max(np.abs(g - r))) <= 5e-5 * float(r.max() - r.min())
+    m.close()
+    ref.close()
+
+
+@pytest.mark.parametrize("nh,nkv,hd,first,n", [(4, 2, 64, 2038, 16), (4, 1, 128, 2038, 16), (8, 1, 64, 2038, 16),
+                                               (8, 1, 128, 2038, 16), (4, 2, 64, 4080, 16)])
+def test_fast_steps_past_one_block_a_chunk(ctx, nh, nkv, hd, first, n):
+    """Steps across position 2048 = 64 x 32, where the chunks of the
+    long-context attention take a second block of 32 positions (and up to the
+    last one, 4095, that a model can have): the next block's request and the
+    running softmax's rescale, in the 512- and the 256-thread forms and both
+    head widths, after a batched prompt. Logits within 5e-5 of the range of the
+    oracle's, the prompt's bound."""
+    cfg = dict(DENSE, n_layers=1, n_heads=nh, n_kv_heads=nkv, head_dim=hd, inter=256, vocab=500, max_pos=first + n)
+    print(f"[gpu] long context: {nh}/{nkv} heads of {hd}, positions {first}..{first + n - 1}", flush=True)
+    m, ref = build(ctx, cfg, 919)
+    m.set_mode(wpcg.MODE_FAST)
+    toks = np.random.default_rng(first + nh).integers(0, cfg["vocab"], first + n).astype(np.uint32)
+    exp = [ref.forward_token(int(t)) for t in toks]
+    m.prefill(toks[:first], want_logits=False)
+    for t, r in zip(toks[first:], exp[first:]):
+        g, _ = m.forward_token(int(t))
         assert float(np.max(np.abs(g - r))) <= 5e-5 * float(r.max() - r.min())
     m.close()
     ref.close()

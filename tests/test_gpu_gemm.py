@@ -235,11 +235,14 @@ def test_gemm_split_every_ksplit(ctx, M):
 # The many-row kernel at the edges of its tiles: one row more than the
 # 64 (SPLIT 32) that k_gemm takes, ragged last tiles of 32 rows of X and of
 # W, odd and even block counts on both sides of the K groups (1, 2, 4, 8), and
-# every workgroup shape (outputs from one tile to more than the chip).
+# every workgroup shape (outputs from one tile to more than the chip;
+# tests/test_wide_shapes.py checks that each shape is among them).
 # 2^-17 and 3e-5 of the term sum as in the bounds above.
 MANY_ROWS = [
     (4, 1, 128, 65), (3, 33, 256, 95), (4, 16, 384, 96), (3, 300, 1152, 129), (4, 700, 1280, 100),
-    (3, 4864, 896, 300), (4, 9728, 640, 500), (3, 2560, 2560, 97), (4, 513, 4224, 1025), (4, 8192, 256, 2080)]
+    (3, 4864, 896, 300), (4, 9728, 640, 500), (3, 2560, 2560, 97), (4, 513, 4224, 1025), (4, 8192, 256, 2080),
+    (4, 15250, 384, 335), (3, 14900, 256, 330), (3, 10950, 384, 131), (4, 11000, 256, 67), (3, 5500, 256, 67),
+    (4, 13210, 256, 131), (3, 11050, 384, 163), (4, 790, 256, 2085), (3, 793, 384, 2085)]
 # and with K in slices over workgroups: long rows of few outputs, an odd count
 # of blocks, a last slice shorter than the others
 K_SLICED = [
@@ -274,3 +277,25 @@ def test_gemm_many_rows(ctx, scheme, rows, cols, M, dtype):
         assert np.array_equal(yd.read(np.float32, M * rows).view(np.uint32), Y.reshape(-1).view(np.uint32))
     lin.close()
     other.close()
+
+
+@pytest.mark.parametrize("scheme", [4, 3])
+@pytest.mark.parametrize("M,dtype", [(100, wpcg.DTYPE_BF16), (65, wpcg.DTYPE_F32), (70, wpcg.DTYPE_F32_SPLIT)])
+def test_gemm_many_rows_with_requested_kslices(ctx, scheme, M, dtype):
+    """With the caller's K-slices a large batch runs in passes of 64 (SPLIT 32)
+    rows: each pass is the bits of a call of its own. Bounds as above."""
+    rows, cols = 300, 128 * 35
+    lin, blocks = make(ctx, scheme, rows, cols, seed=23)
+    X = np.random.default_rng(M).standard_normal((M, cols)).astype(np.float32)
+    bits = to_bf16_bits(X)
+    Xin = bits if dtype == wpcg.DTYPE_BF16 else X
+    split = dtype == wpcg.DTYPE_F32_SPLIT
+    step = 32 if split else 64
+    for kg in (1, 3, 8):
+        lin.set_gemm_kslices(kg)
+        Y = lin.gemm(Xin, dtype)
+        check(Y, X if split else bf16_to_f32(bits), scheme, blocks, rows, cols, TOL_SPLIT if split else TOL_ACC, None,
+              f"M={M} kg={kg}")
+        parts = [lin.gemm(Xin[c:c + step], dtype) for c in range(0, M, step) if min(step, M - c) > 1]
+        assert np.array_equal(np.concatenate(parts).view(np.uint32), Y[:sum(len(q) for q in parts)].view(np.uint32))
+    lin.close()

@@ -101,7 +101,7 @@ def greedy(m, first, steps):
 
 @pytest.mark.parametrize("name,cfg,n_pre,n,seed", [
     ("dense-one-pass", DENSE, 0, 100, 11),
-    ("dense-two-passes", DENSE, 0, 300, 12),
+    ("dense-two-passes", dict(DENSE, max_pos=1100), 0, 1060, 12),
     ("dense-after-steps", DENSE, 7, 90, 13),
     ("moe-one-pass", MOE, 0, 200, 21),
     ("moe-two-passes", MOE, 3, 290, 22),
@@ -174,6 +174,35 @@ def test_fast_prefill_v3_matches_steps(ctx, name, cfg, n, seed):
     print(f"[gpu] prefill {name}: logits {err:.2e} of the steps' range, cache {kerr:.2e}, argmax {got_id} vs "
           f"{ref_id}", flush=True)
     assert err <= TOL and kerr <= TOL and got_id == ref_id
+    m.close()
+
+
+# (query heads, key heads, tokens) that pick each form of the q/k/v launch
+# (tests/test_wide_shapes.py): a workgroup of four heads, of one, of two
+QKV_SHAPES = [(32, 4, 401), (4, 2, 41), (16, 2, 397)]
+
+
+@pytest.mark.parametrize("scheme", [4, 3])
+@pytest.mark.parametrize("nh,nkv,n", QKV_SHAPES)
+def test_fast_prefill_every_qkv_form(ctx, scheme, nh, nkv, n):
+    """The q/k/v launch's norm and rotation in each workgroup shape, a ragged
+    last column group, after 3 steps, against the FAST steps: TOL as above."""
+    cfg = dict(DENSE, n_layers=1, n_heads=nh, n_kv_heads=nkv, head_dim=128, max_pos=416)
+    print(f"[gpu] q/k/v of {nh}/{nkv} heads, {n} tokens, v{scheme}", flush=True)
+    m = wpcg.Model(ctx, scheme, wpcg.ModelConfig(**cfg))
+    for nm, arr in synth.model_tensors(cfg, scheme, 71, wpcg.encode):
+        m.set_tensor(nm, arr)
+    m.set_mode(wpcg.MODE_FAST)
+    toks = np.random.default_rng(n).integers(0, cfg["vocab"], n + 3).astype(np.uint32)
+    for t in toks:
+        ref, ref_id = m.forward_token(int(t))
+    kr, vr = cache(m, cfg, n + 3)
+    m.set_position(3)
+    got, got_id = m.prefill(toks[3:])
+    kg, vg = cache(m, cfg, n + 3)
+    assert float(np.max(np.abs(got - ref))) <= TOL * float(ref.max() - ref.min()) and got_id == ref_id
+    assert float(np.max(np.abs(kg - kr))) <= TOL * float(np.max(np.abs(kr)))
+    assert float(np.max(np.abs(vg - vr))) <= TOL * float(np.max(np.abs(vr)))
     m.close()
 
 

@@ -6,6 +6,7 @@ import subprocess
 
 import pytest
 import test_gpu_gemm
+import test_gpu_prefill
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -32,6 +33,17 @@ def part_floats(rows, nb):
     kg = whole(max(1, min(-(-512 // -(-rows // 128)), nb // 15)))
     small = whole(min(nb, max(min(-(-240 // -(-rows // 64)), max(1, nb // 4)), -(-nb // 30))))
     return max(kg * 64, small * 16) * (-(-rows // 16) * 16) if kg > 1 or small > 1 else 0
+
+
+def test_every_shape_is_covered(pick):
+    seen = {(split, scheme, pick(split, 0, scheme, m, cols, part_floats(rows, cols // 128), [rows])[0])
+            for scheme, rows, cols, m in test_gpu_gemm.MANY_ROWS for split in (0, 1)}
+    assert seen == {(p, s, h) for p in (0, 1) for s in (3, 4) for h in range(5)}
+    # the q/k/v epilogue's forms, each with both schemes
+    qkv = [[nh * 128, nkv * 128, nkv * 128] for nh, nkv, _ in test_gpu_prefill.QKV_SHAPES]
+    for scheme in (3, 4):
+        assert {pick(1, 1, scheme, n, 256, 0, rows)[0] for rows, (_, _, n) in zip(qkv, test_gpu_prefill.QKV_SHAPES)} \
+            == {0, 1, 2}
 
 
 def test_k_slices_where_half_the_chip_idles(pick):
