@@ -180,10 +180,13 @@ int wpcg_linear_matvec_multi(int n, wpcg_linear* const* lins, const float* const
  * X: M rows of in_f values, contiguous, fp32 (x_dtype WPCG_DTYPE_F32) or
  * bf16 bit patterns (WPCG_DTYPE_BF16); Y: M rows of out_f floats. With
  * M == 1 and fp32 X this is wpcg_linear_matvec in the linear's mode. Else
- * the matrix-core kernels run (one up to 64 rows of X, another, every row
- * in one launch, above): the codes are exact, X is rounded to bf16 (exact when given as bf16), each block's
- * dots accumulate in fp32 and its scale and zero point are applied in fp32
- * (the weights are never rounded). The first batched call on a linear
+ * the matrix-core kernels run (one up to 64 rows of X, SPLIT 32; above that
+ * another, every row in one launch): the codes are exact, X is rounded to
+ * bf16 (exact when given as bf16), each block's dots accumulate in fp32 and
+ * its scale and zero point are applied in fp32 (the weights are never
+ * rounded), in an order that depends on the sizes, M among them: the same
+ * call gives the same bits, a row in a batch of another size the same value
+ * within the rounding of those sums. The first batched call on a linear
  * allocates its workspace (about 16 KiB per 128 inputs plus the split-K
  * partials); make it before capturing a graph that contains the call. The
  * first ones with more than 64 rows of X (SPLIT: 32) also allocate a packed
@@ -220,7 +223,8 @@ int wpcg_linear_gemm_noalloc(wpcg_linear* lin, const void* x_dev, int x_dtype, u
                              wpcg_stream stream);
 /* K-slices of the batched kernels (0 = the library's choice; a tuning knob,
  * no reference counterpart), applied to both (M <= 16 and M > 16) within
- * their limits; while it is set, more than 64 rows of X run 64 at a time. Frees the workspace; the next batched call makes it. The
+ * their limits; while it is set, more than 64 rows of X (SPLIT: 32) run 64
+ * (32) at a time. Frees the workspace; the next batched call makes it. The
  * query returns the splits in use (or planned) for M <= 16 and M > 16. */
 int wpcg_linear_set_gemm_kslices(wpcg_linear* lin, int kslices);
 int wpcg_linear_gemm_kslices(wpcg_linear* lin, int* kslices_small, int* kslices);
@@ -469,9 +473,10 @@ int wpcg_model_generate(wpcg_model* m, const uint32_t* prompt, uint32_t n_prompt
  * decode step's device buffers as the last step left them. which: 0
  * residual, 1 normed (after the final norm; EXACT mode), 2 q (the
  * projection), 3 k and 4 v (the last layer's projections), 5 attention
- * output (EXACT mode, and FAST dense models, which merge the attention
- * chunks in a launch of their own; FAST Qwen3-MoE merges them inside
- * o_proj and leaves this buffer unwritten), 7 logits, 9 K cache, 10 V
+ * output (EXACT mode, FAST dense models, and FAST Qwen3-MoE from position
+ * 768 on, which merge the attention chunks in a launch of their own; before
+ * that FAST Qwen3-MoE merges them inside o_proj and leaves this buffer
+ * unwritten), 7 logits, 9 K cache, 10 V
  * cache ([layer][kv_head][max_pos][head_dim]). In FAST dense models whose
  * down projection defers its K-slices to its readers, the residual (0)
  * excludes the last layer's deferred slices: the head adds them as it

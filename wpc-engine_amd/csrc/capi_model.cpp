@@ -675,7 +675,7 @@ int prefill_run(wpcg_model* m, uint32_t pos0, uint32_t n, uint32_t n_prompt)
 
 // FAST verification of tokens[pos0 .. pos0+n-1] (n <= WPCG_VERIFY_MAX <= cap,
 // one pass): every row's logits (final norm, head as one batched GEMM) and
-// argmax; the position ends at pos0 + n with the last argmax as st.last.
+// argmax; the position ends at pos0 + n.
 int verify_run(wpcg_model* m, uint32_t pos0, uint32_t n)
 {
     if (int rc = make_prefill(m, n)) return rc;
@@ -697,7 +697,7 @@ int verify_run(wpcg_model* m, uint32_t pos0, uint32_t n)
     const float* bs[1] = {head->bias};
     WPCG_HIP(launch_gemm_packed_rows(ms, bs, &P.vlogits, 1, P.xf, P.xsum, (int)n, nullptr, s));
     WPCG_HIP(launch_argmax_rows(P.vlogits, (int)c.vocab, (int)n, P.vids, s));
-    // (the state's last token stays the host's business: the caller has every argmax)
+    // (the state's last argmax is left 0: the caller has them all)
     if (int rc = put_state(m, DecodeState{pos0 + n, 0xffffffffu, c.max_pos, 0}, nullptr, 0)) return rc;
     return WPCG_OK;
 }

@@ -14,7 +14,10 @@ namespace wpcg {
 // X; the shape with the fewest rounds x time wins. Large outputs fill the
 // chip with the widest tile (15360 x 3840, 1024 rows: 256 x 128 144 us,
 // 128 x 64 164, 64 x 32 357), small ones need the narrow, K-split ones
-// (3840 x 15360, 128 rows: 64 x 32 37 us, 128 x 64 97, 256 x 128 197).
+// (3840 x 15360, 128 rows: 64 x 32 37 us, 128 x 64 97, 256 x 128 197). The
+// 16-wave forms are held to 128 registers and some spill, which their costs
+// contain (registers spilled, v4 and v3: SPLIT 128 x 32 10 and 16, its q/k/v
+// form 0 and 11, SPLIT 128 x 64 18 and 21, 64 x 32 8 and 18).
 struct WideShape {
     int rows32, cols32;
     int cost[2];
