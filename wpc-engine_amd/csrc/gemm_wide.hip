@@ -22,10 +22,10 @@
 // of 64 x 64 outputs each took 158-171 us, two groups of waves alternating
 // between vector and matrix phases 160-197.
 //
-// Measured, us a call, before -> now: 15360 x 3840 v4 at 1024 rows of bf16
-// 384 -> 128, 9728 x 2560 v3 at 777 rows SPLIT 541 -> 84; in the prefill
-// (Qwen3-4B shape, 1000 tokens, per layer) gate and up 350 -> 208, q/k/v
-// 142 -> 76, o and down 310 -> 200.
+// Measured, us a call, before -> now (two cards): 15360 x 3840 v4 at 1024 rows
+// of bf16 383-396 -> 128-135, 9728 x 2560 v3 at 777 rows SPLIT 541 -> 84-91;
+// in the prefill (Qwen3-4B shape, 1000 tokens, per layer) gate and up 350 ->
+// 208, q/k/v 142 -> 76, o and down 310 -> 200.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
