@@ -46,7 +46,7 @@ def test_every_shape_is_covered(pick):
             == {0, 1, 2}
 
 
-def test_k_slices_where_half_the_chip_idles(pick):
+def test_k_slices_where_the_chip_has_room(pick):
     """The sliced cases of the GPU tests are sliced (both shapes, both
     schemes, both kinds of X), the others are not; no slice is empty; nothing
     is sliced without the workspace for it."""

@@ -37,13 +37,15 @@ constexpr WideShape WIDE_SPLIT[] = {{16, 1, {160, 165}, false, false},
                                     {2, 1, {60, 70}, false, true},
                                     {4, 2, {100, 110}, false, false}};
 
-// K-slices over workgroups, for launches that leave half of the chip idle
-// even in 64 x 32 tiles (SPLIT 3840 x 15360 v3, 96 rows, 180 such tiles: 49.4
-// us without slices, 52.9 with; 512 x 12288, 24 tiles: 43.2, 24.4):
+// K-slices over workgroups, where the chip has room for all of them at once:
 // slices of at least WIDE_SLICE blocks, whose partials cost a second launch
 // (k_gemm_reduce, 4.1-4.8 us in a trace, and the gap before it), their way
 // through memory, and the start of a short run of blocks (a quarter more a
-// block).
+// block). Up to 256 of the 64 x 32 tiles (us without and with: 2560 x 9728 v3,
+// 160, bf16 100 rows 31.9 and 25.1; 3840 x 15360 v3, 180, bf16 65 rows 44.6
+// and 34.6), SPLIT up to 128 of them (512 x 12288 v3, 24, 96 rows 43.2 and
+// 24.4; but 3840 x 15360, 180, 96 rows v3 49.4 and 52.9, v4 with the weights
+// in HBM 49.1 and 53.5).
 constexpr int WIDE_SLICE = 8;
 constexpr int64_t WIDE_REDUCE = 550;            // hundredths of a microsecond
 constexpr int64_t WIDE_PART_FLOATS = 5000;      // partial sums written and read in one of those
@@ -63,7 +65,7 @@ inline WidePick pick_wide(bool split, bool rope, int scheme, const int* tiles32,
     const int n = rope ? 3 : 5;
     int64_t small = 0;  // 64 x 32 tiles
     for (int e = 0; e < nmat; e++) small += (int64_t)((tiles32[e] + 1) / 2) * cols32;
-    const int most = rope || nmat > 1 || small > 128
+    const int most = rope || nmat > 1 || small > (split ? 128 : 256)
                          ? 1
                          : (int)std::min<uint64_t>(part_floats / std::max<uint64_t>(outs, 1),
                                                                      (uint64_t)std::max(nb / WIDE_SLICE, 1));
