@@ -124,7 +124,7 @@ __device__ __forceinline__ bf16x8 codes_bf16(uint32_t a, uint32_t b)
 // weight rows and 24 rows of X are 40 workgroups of the smallest shape): each
 // takes a run of blocks and leaves its sums in part, which the next launch
 // (launch_gemm_reduce) adds in slice order: o_proj and down of a 24-token
-// Qwen3-4B-shaped prompt 51.6 us together without slices, 24.3 and 8.8 for the
+// Qwen3-4B-shaped prompt 51.6 us together without slices, 20.1 and 8.2 for the
 // reduces with them; 512 x 12288 at 33 rows SPLIT 39.6 -> 23.7 us a call. (A
 // form of its own: with the slice in the other launches too, the small v3
 // ones were 1 us slower.)
@@ -452,7 +452,7 @@ hipError_t launch_any(WideArgs& a, uint32_t M, bool rope, float* part, uint64_t 
             return p.shape == 3 ? launch_cfg<SCHEME, SPLIT, 1, 4, 1, 4, false, true>(a, s)
                                 : launch_cfg<SCHEME, SPLIT, 1, 2, 1, 8, false, true>(a, s);
         else
-            return p.shape == 1 ? launch_cfg<SCHEME, SPLIT, 1, 4, 1, 4, false, true>(a, s)
+            return p.shape == 1 ? launch_cfg<SCHEME, SPLIT, 1, 4, 1, 2, false, true>(a, s)
                                 : launch_cfg<SCHEME, SPLIT, 1, 2, 1, 4, false, true>(a, s);
     }
     if constexpr (!SPLIT) {
@@ -467,13 +467,13 @@ hipError_t launch_any(WideArgs& a, uint32_t M, bool rope, float* part, uint64_t 
         if (rope) {
             switch (p.shape) {
             case 0: return launch_cfg<SCHEME, SPLIT, 1, 16, 1, 1, true>(a, s);
-            case 1: return launch_cfg<SCHEME, SPLIT, 1, 4, 1, 4, true>(a, s);
+            case 1: return launch_cfg<SCHEME, SPLIT, 1, 4, 1, 2, true>(a, s);
             default: return launch_cfg<SCHEME, SPLIT, 1, 8, 1, 2, true>(a, s);
             }
         }
         switch (p.shape) {
         case 0: return launch_cfg<SCHEME, SPLIT, 1, 16, 1, 1>(a, s);
-        case 1: return launch_cfg<SCHEME, SPLIT, 1, 4, 1, 4>(a, s);
+        case 1: return launch_cfg<SCHEME, SPLIT, 1, 4, 1, 2>(a, s);
         case 2: return launch_cfg<SCHEME, SPLIT, 1, 8, 1, 2>(a, s);
         case 3: return launch_cfg<SCHEME, SPLIT, 1, 2, 1, 4>(a, s);
         default: return launch_cfg<SCHEME, SPLIT, 1, 4, 2, 2>(a, s);

@@ -16,8 +16,12 @@ namespace wpcg {
 // 128 x 64 164, 64 x 32 357), small ones need the narrow, K-split ones
 // (3840 x 15360, 128 rows: 64 x 32 37 us, 128 x 64 97, 256 x 128 197). The
 // 16-wave forms are held to 128 registers and some spill, which their costs
-// contain (registers spilled, v4 and v3: SPLIT 128 x 32 10 and 16, its q/k/v
-// form 0 and 11, SPLIT 128 x 64 18 and 21, 64 x 32 8 and 18).
+// contain (registers spilled, v4 and v3: SPLIT 128 x 64 18 and 21, 64 x 32 8
+// and 18). SPLIT 128 x 32 has two K groups in 8 waves: with four in 16 waves,
+// whose cost this is, it spilled 10 and 16 and took a tenth to a quarter longer
+// wherever it is picked (9728 x 2560 at 33 rows, weights in HBM: v4 22.9 us,
+// now 18.3, v3 27.6 and 20.9; gate and up of a 24-token Qwen3-4B-shaped prompt
+// 22.7 and 17.2).
 struct WideShape {
     int rows32, cols32;
     int cost[2];
@@ -41,11 +45,10 @@ constexpr WideShape WIDE_SPLIT[] = {{16, 1, {160, 165}, false, false},
 // slices of at least WIDE_SLICE blocks, whose partials cost a second launch
 // (k_gemm_reduce, 4.1-4.8 us in a trace, and the gap before it), their way
 // through memory, and the start of a short run of blocks (a quarter more a
-// block). Up to 256 of the 64 x 32 tiles (us without and with: 2560 x 9728 v3,
-// 160, bf16 100 rows 31.9 and 25.1; 3840 x 15360 v3, 180, bf16 65 rows 44.6
-// and 34.6), SPLIT up to 128 of them (512 x 12288 v3, 24, 96 rows 43.2 and
-// 24.4; but 3840 x 15360, 180, 96 rows v3 49.4 and 52.9, v4 with the weights
-// in HBM 49.1 and 53.5).
+// block). Up to 256 of the 64 x 32 tiles; us without and with: 512 x 12288 v3,
+// 24 tiles, SPLIT 96 rows 43.2 and 24.4; 2560 x 9728 v3, 160, bf16 100 rows
+// 31.9 and 25.1, SPLIT 37.5 and 29.4; 3840 x 15360 v3, 180, bf16 65 rows 44.6
+// and 34.6, SPLIT 96 rows 49.4 and 43.8.
 constexpr int WIDE_SLICE = 8;
 constexpr int64_t WIDE_REDUCE = 550;            // hundredths of a microsecond
 constexpr int64_t WIDE_PART_FLOATS = 5000;      // partial sums written and read in one of those
@@ -65,7 +68,7 @@ inline WidePick pick_wide(bool split, bool rope, int scheme, const int* tiles32,
     const int n = rope ? 3 : 5;
     int64_t small = 0;  // 64 x 32 tiles
     for (int e = 0; e < nmat; e++) small += (int64_t)((tiles32[e] + 1) / 2) * cols32;
-    const int most = rope || nmat > 1 || small > (split ? 128 : 256)
+    const int most = rope || nmat > 1 || small > 256
                          ? 1
                          : (int)std::min<uint64_t>(part_floats / std::max<uint64_t>(outs, 1),
                                                                      (uint64_t)std::max(nb / WIDE_SLICE, 1));
