@@ -192,8 +192,9 @@ int wpcg_linear_matvec_multi(int n, wpcg_linear* const* lins, const float* const
  * first ones with more than 64 rows of X (SPLIT: 32) also allocate a packed
  * X: 2 bytes (SPLIT: 4) an input for each row of X, the rows rounded up to
  * 128, 256, ... 2048 (SPLIT: half of that) and at most 2048 (1024) of them.
- * Captured before that, or where it cannot be allocated, such a call runs in
- * passes of fewer rows (64, SPLIT 32, without any), with the same result.
+ * They may be captured: the array is the linear's, like its workspace. Where
+ * it cannot be allocated, such a call runs in passes of fewer rows (64, SPLIT
+ * 32, without any), with the same result.
  * WPCG_DTYPE_F32_SPLIT: fp32 X fed to the matrix cores as two bf16 terms
  * hi = bf16(x), lo = bf16(x - hi), so X is carried to a relative 2^-18
  * (twice the matrix-core work). */

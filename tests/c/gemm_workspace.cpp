@@ -1,7 +1,7 @@
 // The workspace rules of the batched GEMM (csrc/capi_gemm.cpp) with the HIP
 // calls and kernel launchers replaced by counters: how much a call allocates,
-// what it falls back to when an allocation fails or a graph is captured, and
-// that what a captured graph may hold stays allocated. Then the rows of the
+// captured or not, what it falls back to when an allocation fails, and that
+// what a captured graph may hold stays allocated. Then the rows of the
 // prefill's batch buffers (grow_rows).
 #include "../../wpc-engine_amd/csrc/capi_gemm.cpp"
 
@@ -12,6 +12,8 @@
 static std::map<void*, size_t> live;
 static size_t held, limit = ~size_t(0);
 static bool capturing, pending;
+static hipStreamCaptureMode mode = hipStreamCaptureModeGlobal;
+static int broken;  // captures that an allocation ended
 struct Launch {
     void* xf;
     float* xsum;
@@ -24,6 +26,10 @@ static int passes;
 extern "C" {
 hipError_t hipMalloc(void** p, size_t n)
 {
+    if (capturing && mode != hipStreamCaptureModeRelaxed) {
+        broken++;
+        return hipErrorStreamCaptureUnsupported;
+    }
     if (held + n > limit) {
         pending = true;
         return hipErrorOutOfMemory;
@@ -49,6 +55,11 @@ hipError_t hipGetLastError()
 hipError_t hipMemsetAsync(void*, int, size_t, hipStream_t) { return hipSuccess; }
 hipError_t hipMemcpyAsync(void*, const void*, size_t, hipMemcpyKind, hipStream_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode* m)
+{
+    std::swap(*m, mode);
+    return hipSuccess;
+}
 hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* st)
 {
     *st = capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
@@ -142,17 +153,21 @@ int main()
         free_gemm(L.gemm);
         CHECK(held == 0);
     }
-    {  // captured: nothing is allocated
+    {  // captured: as outside, with the capture's mode as it was afterwards
         wpcg_linear L{};
         linear(L);
         CHECK(gemm(L, bf, 2) == WPCG_OK);
         capturing = true;
         const size_t base = held;
-        CHECK(gemm(L, bf, 500) == WPCG_OK && launched[0].tiles == 4 && held == base);
-        capturing = false;
-        CHECK(gemm(L, bf, 200) == WPCG_OK && launched[0].tiles == 16);
-        capturing = true;
-        CHECK(gemm(L, bf, 500) == WPCG_OK && launched[0].tiles == 16 && held == base + packed(16));
+        CHECK(gemm(L, bf, 500) == WPCG_OK && launched[0].tiles == 32 && held == base + packed(32));
+        CHECK(broken == 0 && mode == hipStreamCaptureModeGlobal);
+        limit = held;
+        CHECK(gemm(L, bf, 600) == WPCG_OK && launched[0].tiles == 32 && broken == 0 && !pending);
+        CHECK(mode == hipStreamCaptureModeGlobal);
+        limit = ~size_t(0);
+        wpcg_linear N{};  // the first batched call on a linear is still refused
+        linear(N);
+        CHECK(gemm(N, bf, 500) == WPCG_E_ARG && launched.empty() && broken == 0);
         capturing = false;
         free_gemm(L.gemm);
     }

@@ -1,7 +1,7 @@
 """The batched GEMM's workspace on the host (tests/c/gemm_workspace.cpp, which
 includes csrc/capi_gemm.cpp and counts the allocations and launches): sized to
-the call, and a call that cannot have it, or is being captured, runs on what
-is there instead of failing; and how many rows the prefill's buffers get."""
+the call, captured or not, and a call that cannot have it runs on what is there
+instead of failing; and how many rows the prefill's buffers get."""
 import os
 import subprocess
 

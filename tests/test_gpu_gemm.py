@@ -264,7 +264,7 @@ def test_gemm_many_rows(ctx, scheme, rows, cols, M, dtype):
     check(Y, X if split else bf16_to_f32(bits), scheme, blocks, rows, cols, TOL_SPLIT if split else TOL_ACC, bias,
           f"M={M}")
     assert np.array_equal(Y.view(np.uint32), lin.gemm(bits if dtype == wpcg.DTYPE_BF16 else X, dtype).view(np.uint32))
-    # captured before the packed X of this size exists: smaller passes, the same bits
+    # captured before the packed X of this size exists: made there, the same bits
     other, _ = make(ctx, scheme, rows, cols, rows + cols, bias)
     xd = ctx.upload(bits if dtype == wpcg.DTYPE_BF16 else X)
     yd = ctx.alloc(4 * M * rows)
