@@ -208,7 +208,8 @@ int wpcg_linear_gemm_host(wpcg_linear* lin, const void* x, int x_dtype, uint32_t
 /* wpcg_linear_gemm that allocates nothing: the same kernels, splits and
  * results (bit for bit), with the workspace (packed X, per-block column
  * sums, split-K partials, counters) carved from a fixed device array of
- * WPCG_NOALLOC_SCRATCH_BYTES that the library holds on each GPU it runs on
+ * WPCG_NOALLOC_SCRATCH_BYTES (and 64 MiB more for the packed X of more than
+ * 64 rows, SPLIT 32) that the library holds on each GPU it runs on
  * until the process ends, instead of the linear's own workspace. No
  * reference counterpart: for callers that cannot allocate device memory
  * (code under HIP graph capture, serving loops, harnesses that forbid

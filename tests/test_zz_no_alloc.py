@@ -86,6 +86,8 @@ def test_two_calls_in_a_row_second_smaller(ctx):
     (4, 2560, 9728, 130, wpcg.DTYPE_BF16),       # the same, one row tile more than 64 rows take
     (3, 512, 12288, 90, wpcg.DTYPE_BF16),        # K-slices over workgroups
     (4, 2560, 9728, 40, wpcg.DTYPE_F32_SPLIT),   # the same
+    (4, 48, 51200, 645, wpcg.DTYPE_BF16),        # more rows than the array holds packed: two passes
+    (3, 48, 51200, 330, wpcg.DTYPE_F32_SPLIT),   # the same
     (3, 4096, 2560, 16, wpcg.DTYPE_BF16),        # the small kernel
     (4, 3840, 15360, 64, wpcg.DTYPE_BF16),       # Gemma-12B down_proj (config 4)
     (4, 4864, 896, 1, wpcg.DTYPE_F32),           # M = 1 fp32: the matvec

@@ -197,10 +197,11 @@ int wpcg_linear_gemm_noalloc(wpcg_linear* L, const void* x, int x_dtype, uint32_
     w.xsum = reinterpret_cast<float*>(base + o_xsum);
     w.xf = base + o_xf;
     w.part = part ? reinterpret_cast<float*>(base + o_part) : nullptr;
-    if (wide(L, x_dtype, M)) {  // as many 16-column tiles as the array holds packed, a multiple of 4
-        const uint64_t room = WPCG_NOALLOC_SCRATCH_BYTES - o_xsum;
-        const int tiles = (int)std::min<uint64_t>(GEMM_WIDE_TILES, room / (m.nb * (4096 + 64)) / 4 * 4);
-        w.xf = base + o_xsum + up(m.nb * tiles * 64);
+    if (wide(L, x_dtype, M)) {  // packed X behind the rest; its sums need half of what xf would take there
+        const int tiles = (int)std::min<uint64_t>(GEMM_WIDE_TILES, SCRATCH_PACK_BYTES / (m.nb * 4096) / 4 * 4);
+        static_assert(SCRATCH_PACK_BYTES >= 4 * WPCG_NOALLOC_SCRATCH_BYTES && GEMM_WIDE_TILES * 64 <= 4 * 4096,
+                      "four tiles at least, and room for the sums of all");
+        w.xf = base + WPCG_NOALLOC_SCRATCH_BYTES;
         WPCG_HIP(launch_gemm_wide(m, w.xf, w.xsum, tiles, x, x_dtype, M, L->bias, y, w.part, part_floats(m, w), s));
         return WPCG_OK;
     }

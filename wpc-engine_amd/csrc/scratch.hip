@@ -15,7 +15,7 @@
 
 #include "wpcg_internal.hpp"
 
-static __device__ __align__(256) unsigned char scratch[WPCG_NOALLOC_SCRATCH_BYTES];
+static __device__ __align__(256) unsigned char scratch[WPCG_NOALLOC_SCRATCH_BYTES + wpcg::SCRATCH_PACK_BYTES];
 
 namespace wpcg {
 namespace {

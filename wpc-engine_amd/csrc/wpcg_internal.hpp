@@ -303,8 +303,13 @@ hipError_t launch_gemm_grouped(const DeviceMatrix& m, const DeviceMatrix* m2, co
 // scratch_setup(device) looks up the device address of the library's fixed
 // workspace array on `device` (which must be current) and keeps it;
 // wpcg_ctx_create runs it. scratch_ptr(device) returns that address (null
-// before set-up). launch_fill_u32 writes v to p[0..n) with a kernel (no
+// before set-up): WPCG_NOALLOC_SCRATCH_BYTES, then SCRATCH_PACK_BYTES for the
+// many-row GEMM's packed X (2048 rows of 15360 bf16 inputs in one pass; in
+// the first array alone, passes of ever fewer rows the longer a row is, and
+// 1024 rows of 1024 x 40960 SPLIT took 2246 us where passes of 32 with the
+// kernels up to that size took 1077). launch_fill_u32 writes v to p[0..n) with a kernel (no
 // memset node, so a captured graph replays it correctly).
+constexpr uint64_t SCRATCH_PACK_BYTES = 64u << 20;
 int scratch_setup(int device);
 void* scratch_ptr(int device);
 hipError_t launch_fill_u32(uint32_t* p, int n, uint32_t v, hipStream_t s);
